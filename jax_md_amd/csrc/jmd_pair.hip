@@ -36,8 +36,8 @@ JMD_DENSE_INSTANCES(JMD_DENSE_EXTERN)
 // LDS hash table and adds each entry to memory once.  A receiver that finds
 // no free slot within kProbe probes goes to memory directly.  Any pair order
 // is correct; ordered lists only make the sums shorter.
-constexpr int kSparseChunk = JMD_SPARSE_CHUNK;  // pairs per workgroup pass
-constexpr int kSparseTable = JMD_SPARSE_TABLE;  // LDS hash entries (power of two)
+constexpr int kSparseChunk = 4096;  // pairs per workgroup pass
+constexpr int kSparseTable = 2048;  // LDS hash entries (power of two)
 constexpr int kProbe = 16;
 
 template <int DIM, int STRIDE, int KIND, bool GENERAL, bool ENERGY>
@@ -216,6 +216,22 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
 }
 
 static int g_tpa_override = 0;
+
+// Lanes per Dense row.  3-D rows get 8 lanes once the rows fill the chip; a
+// smaller system has too few wavefronts for that, and a row's own chain of
+// loads decides, so its entries are spread over more lanes, as far as the
+// rows are long enough to feed them.  A 20-step block of Lennard-Jones rows
+// of 95 entries, us with 8 / 16 / 32 lanes: 330 / 293 / 278 (N = 4,096),
+// 330 / 299 / 296 (8,000), 375 / 361 / 384 (15,625), 417 / 408 / 441 (22,736),
+// 463 / 478 / 519 (32,768).  2-D rows (a few entries) get 2.
+static int lanes_per_row(int dim, int64_t n, int64_t width) {
+  if (g_tpa_override) return g_tpa_override;
+  if (dim == 2) return 2;
+  if (n <= 8192 && width >= 64) return 32;
+  if (n <= 24576 && width >= 32) return 16;
+  return 8;
+}
+
 constexpr long long kSparseBlocks = 2048;
 
 // Virial W_ab = weight sum over the list's ordered pairs of (U'(r)/r) d_a d_b
@@ -384,8 +400,8 @@ using namespace jmd;
 extern "C" {
 
 size_t jmd_pair_workspace_bytes(int64_t n) {
-  // block partials: Dense uses at most ceil(n*16/256) padded to 8, Sparse at
-  // most kSparseBlocks.
+  // block partials: Dense uses at most ceil(n*16/256) padded to 8 (32 lanes a
+  // row only up to n = 8192, 1024 blocks), Sparse at most kSparseBlocks.
   long long blocks = (n * 16 + 255) / 256 + 64;
   if (blocks < kSparseBlocks) blocks = kSparseBlocks;
   return (size_t)(blocks * 8 + 256);
@@ -437,7 +453,7 @@ int pair_energy_force(const float* position, int64_t n, int32_t dim, int32_t pos
       }
       return JMD_OK;
     }
-    int tpa = g_tpa_override ? g_tpa_override : (dim == 3 ? 8 : 2);
+    const int tpa = lanes_per_row(dim, n, idx_width);
     long long threads = (long long)nn * tpa;
     int nb = ceil_div(threads, 256);
     nb = (nb + 7) & ~7;
@@ -627,7 +643,7 @@ int jmd_nve_force_kick_drift(const float* position, int64_t n, int32_t dim,
   box_inverse(kd.s, kd.Ti);
   hipStream_t st = (hipStream_t)stream;
   const int nn = (int)n;
-  const int tpa = g_tpa_override ? g_tpa_override : (dim == 3 ? 8 : 2);
+  const int tpa = lanes_per_row(dim, n, idx_width);
   int nb = ceil_div((long long)nn * tpa, 256);
   nb = (nb + 7) & ~7;
   DenseLaunch L{dim3(nb), st, position, nn, s, a, idx, (int)idx_width, force, nullptr,

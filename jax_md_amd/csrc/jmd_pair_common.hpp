@@ -19,7 +19,7 @@ struct PairArgs {
   const int* species;
   int ns;
   float ro2, rc2, inv_d;  // LJ smoothing: r_on^2, r_c^2, 1/(rc^2-ro^2)^3
-  float c1;               // rc^2 - 3 ro^2
+  float sw, sw_rc2, sw2;  // 1/(rc^2-ro^2), rc^2/(rc^2-ro^2), 2/(rc^2-ro^2)
   float ro;               // LJ r_on
   int smooth;             // r_on < r_c
   float rc;               // interaction range (LJ r_c, soft sphere max sigma)
@@ -49,6 +49,40 @@ __device__ __forceinline__ float fast_rsqrt(float x) {
   return fmaf(y, e, y);
 }
 
+// Switched Lennard-Jones from r^2 and sigma^2, without the factors of
+// epsilon: returns g = -U'/(24 eps r) and *v = U/(4 eps).  With
+// t = (sigma^2/r^2)^3, A = t - 1, B = 2 t - 1 and, for the switch,
+//   y = clamp((rc^2 - r^2) / (rc^2 - ro^2), 0, 1),  x = 1 - y,
+//   S = y^2 (3 - 2 y),  S'/r = -12 x y / (rc^2 - ro^2):
+//   v = S t A,  g = t y [ y (3 - 2 y) B / r^2 + 2 x A / (rc^2 - ro^2) ].
+// The clamp covers all three regions (y = 1: plain, y = 0: beyond the
+// cutoff) and costs nothing on the multiply-add; the common factor t y is
+// taken out, so a pair is 17 operations from r^2 to g.  The caller applies
+// the factors once per row where epsilon is one number.
+// v_rcp_f32 alone (1 ulp): a Newton step moved the force error against FP64
+// by under 5% and cost two operations per pair.
+template <int SMOOTH>
+__device__ __forceinline__ float lj_reduced(float r2, float sig2, const PairArgs& a, float* v) {
+#pragma clang fp contract(off)
+  const float inv_r2 = __builtin_amdgcn_rcpf(r2);
+  const float s2 = sig2 * inv_r2;
+  const float t = s2 * s2 * s2;
+  const float B = fmaf(2.0f, t, -1.0f);
+  if (SMOOTH == 1 || (SMOOTH < 0 && a.smooth)) {
+    const float y = __builtin_amdgcn_fmed3f(fmaf(r2, -a.sw, a.sw_rc2), 0.0f, 1.0f);
+    const float x = 1.0f - y;
+    const float z = y * fmaf(-2.0f, y, 3.0f);
+    const float A2 = fmaf(t, a.sw2, -a.sw2);  // 2 A / (rc^2 - ro^2)
+    const float q = fmaf(z, B * inv_r2, x * A2);
+    const float ty = t * y;
+    *v = z * ty * (t - 1.0f);
+    return q * ty;
+  }
+  const bool valid = r2 < a.rc2;
+  *v = valid ? t * (t - 1.0f) : 0.0f;
+  return valid ? t * (B * inv_r2) : 0.0f;
+}
+
 // U(r) and dU/dr / r for one pair from r^2, without branches; callers mask
 // invalid lanes with a select.  Multiply-adds are explicit (contraction off)
 // so every kernel variant rounds alike.
@@ -57,36 +91,10 @@ __device__ __forceinline__ float pair_eval(float r2, float sig, float eps, float
                                            const PairArgs& a, float* dEr) {
 #pragma clang fp contract(off)
   if (KIND == JMD_LENNARD_JONES) {
-    // With t = sigma^2 / r^2, Vp = t^6 - t^3 (V = 4 eps Vp) and
-    // Wp = 2 t^6 - t^3 (V'/r = -24 eps Wp / r^2).  The smoothing factor is
-    // evaluated at rr = r^2 clamped to [ro^2, rc^2] (one med3): S(rr) = 1
-    // below r_on and 0 beyond r_c, and S'(rr) = 0 at both ends, so one
-    // branch-free expression covers all three regions and the cutoff:
-    //   u = rc^2 - rr, q = ro^2 - rr, p = rc^2 + 2 rr - 3 ro^2,
-    //   S = u^2 p / D,  S'/r = 12 u q / D,   D = (rc^2 - ro^2)^3,
-    //   (S V)'/r = 24 eps u (2 q Vp - u p Wp / r^2) / D.
-    // Below r_on this is -24 eps Wp / r^2 up to the rounding of u^2 p / D.
-    // v_rcp_f32 alone (1 ulp): the Newton step moved the force error
-    // against FP64 by under 5% and cost two operations per pair
-    const float inv_r2 = __builtin_amdgcn_rcpf(r2);
-    const float s2 = sig * sig * inv_r2;
-    const float s6 = s2 * s2 * s2;
-    const float s12 = s6 * s6;
-    const float Vp = s12 - s6;
-    const float Wp = fmaf(2.0f, s12, -s6);
-    if (SMOOTH == 1 || (SMOOTH < 0 && a.smooth)) {
-      const float rr = __builtin_amdgcn_fmed3f(r2, a.ro2, a.rc2);
-      const float u = a.rc2 - rr;
-      const float q = a.ro2 - rr;
-      const float pp = fmaf(2.0f, rr, a.c1);
-      const float t2 = u * pp * Wp * inv_r2;
-      const float inner = fmaf(2.0f, q * Vp, -t2);
-      *dEr = 24.0f * eps * a.inv_d * u * inner;
-      return 4.0f * eps * a.inv_d * (u * u * pp) * Vp;
-    }
-    const bool valid = r2 < a.rc2;
-    *dEr = valid ? -24.0f * eps * Wp * inv_r2 : 0.0f;
-    return valid ? 4.0f * eps * Vp : 0.0f;
+    float v;
+    const float g = lj_reduced<SMOOTH>(r2, sig * sig, a, &v);
+    *dEr = -24.0f * eps * g;
+    return 4.0f * eps * v;
   } else {
     // soft sphere: eps/alpha (1 - r/sigma)^alpha for r < sigma
     float inv_r = fast_rsqrt(r2);
@@ -102,10 +110,38 @@ __device__ __forceinline__ float pair_eval(float r2, float sig, float eps, float
   }
 }
 
+// A lane's value from the lane `CTRL` names within its row of 16 lanes (a
+// data-parallel-primitive move: one VALU instruction per 32 bits, no LDS).
+template <int CTRL>
+__device__ __forceinline__ int dpp_move(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_from(float v) {
+  return __int_as_float(dpp_move<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_from(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)dpp_move<CTRL>((int)(unsigned)b);
+  const unsigned hi = (unsigned)dpp_move<CTRL>((int)(unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Sum over groups of TPA consecutive lanes, in every lane of the group.
+// Within a row of 16 lanes the partners come by DPP: the other lane of a
+// pair and the other pair of a quad (quad permutations), then the mirrored
+// lane of 8 and of 16, whose quads (octets) hold their whole sum by then.
+// (Through ds_bpermute the three sums of a step-kernel row cost 18 LDS
+// instructions and their address arithmetic.)
 template <int TPA, typename T>
 __device__ __forceinline__ T group_sum(T v) {
+  if (TPA >= 2) v += dpp_from<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  if (TPA >= 4) v += dpp_from<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  if (TPA >= 8) v += dpp_from<0x141>(v);  // row_half_mirror
+  if (TPA >= 16) v += dpp_from<0x140>(v); // row_mirror
 #pragma unroll
-  for (int off = TPA / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  for (int off = 16; off < TPA; off <<= 1) v += __shfl_xor(v, off, kWave);
   return v;
 }
 
@@ -158,10 +194,13 @@ inline bool make_pair_args(const jmd_pair_potential* p, PairArgs* a) {
   }
   a->smooth = p->kind == JMD_LENNARD_JONES && ro < rc;
   a->inv_d = 0.0f;
-  a->c1 = fmaf(-3.0f, a->ro2, a->rc2);
+  a->sw = a->sw_rc2 = a->sw2 = 0.0f;
   if (a->smooth) {
     double dd = (double)a->rc2 - (double)a->ro2;
     a->inv_d = (float)(1.0 / (dd * dd * dd));
+    a->sw = (float)(1.0 / dd);
+    a->sw_rc2 = (float)((double)a->rc2 / dd);
+    a->sw2 = (float)(2.0 / dd);
   }
   return true;
 }

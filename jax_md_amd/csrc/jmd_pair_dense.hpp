@@ -8,133 +8,196 @@
 
 namespace jmd {
 
+// Rows of a position table through a buffer descriptor whose stride is the
+// row: the load takes the row index itself (no address arithmetic), and an
+// index of n or more reads zeros.  The intrinsics have no clang builtin, so
+// they are bound by name.
+typedef int rsrc_t __attribute__((ext_vector_type(4)));
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef float f3_t __attribute__((ext_vector_type(3)));
+__device__ f3_t struct_load3(rsrc_t rsrc, int index, int voffset, int soffset,
+                             int aux) __asm("llvm.amdgcn.struct.buffer.load.v3f32");
+__device__ f2_t struct_load2(rsrc_t rsrc, int index, int voffset, int soffset,
+                             int aux) __asm("llvm.amdgcn.struct.buffer.load.v2f32");
+
+__device__ __forceinline__ rsrc_t row_table(const float* p, unsigned rows, int row_bytes) {
+  const unsigned long long b = (unsigned long long)p;
+  return rsrc_t{(int)(unsigned)b, (int)((unsigned)(b >> 32) & 0xffffu) | (row_bytes << 16),
+                (int)rows, 0x00020000};
+}
+
 // Sum over one Dense row slice (entries sub, sub+TPA, ...) into f, e.
-// INTERIOR: every particle of the wavefront lies at least the interaction
-// range from each box face, so for any pair within range the plain
-// difference x_j - x_i is already the minimum image and no wrap is needed
-// (pairs whose plain difference is not the minimum image are then beyond
-// range and contribute zero either way).
-template <int DIM, int STRIDE, int KIND, int TPA, bool GENERAL, bool ENERGY, bool INTERIOR,
-          int SMOOTH, bool BOX = false>
+//
+// What bounds it: the gathers, then VALU issue.  A list at r_c + skin = 3.0
+// holds 95 entries a row at rho 0.8442; at N = 262,144 the L1 serves 22 M
+// requests a launch (86 k of 115 k cycles on each CU) and each SIMD issues
+// 80 k cycles of VALU work, 35 operations a pair and 26 of them the pair's
+// own.  (Timing copies: without half of the arithmetic 1.5 us of 49 less, with
+// neighbours that are consecutive rows 12 us less.  16-byte loads of the
+// entries saved a third of the load instructions and made the gathers' L1
+// requests 15% more; two blocks of entries in flight changed nothing.)
+// * Folds are decided per block of UNR entries and dimension: while every
+//   plain difference of the block is shorter than half the side, it is the
+//   minimum image, and a maximum and a ballot replace the selects.  `near`
+//   (bit c, wavefront-uniform) is clear where no row of the wavefront lies
+//   within the interaction range of a face of dimension c and every position
+//   lies in the box: pairs in range then need no fold and the others add
+//   zero either way.  (Before, wavefronts near any face, 22% of them at
+//   N = 262,144 and all of them when the positions were not known to lie in
+//   the box, folded every component of every pair.)
+// * In a block whose entries are valid in every lane no entry needs a mask;
+//   the masked form runs in the block where some row of the wavefront ends.
+// * Constant factors of the potential are applied once per row (lj_reduced).
+// * INDEXED gathers (tables below 2 GiB) go through row_table.
+// Step kernel at N = 262,144: 48.4 -> 45 us; energy and force of 1,029,897
+// particles not known to lie in the box: 202 -> 176 us.
+template <int DIM, int STRIDE, int KIND, int TPA, bool GENERAL, bool ENERGY, int SMOOTH,
+          bool BOX, bool INDEXED, int UNR>
 __device__ __forceinline__ void row_sum(const float* __restrict__ pos, unsigned n,
                                         const Space& s, const PairArgs& a,
                                         const int* __restrict__ row, int width, int sub,
-                                        unsigned i, const float* xi, const float* xim,
-                                        float* f, float* e) {
+                                        unsigned i, const float* xi, unsigned near, float* f,
+                                        float* e) {
 #pragma clang fp contract(off)
+  constexpr bool LJ = KIND == JMD_LENNARD_JONES;
   float sig = a.sig, eps = a.eps, alp = a.alp;
+  const float sig2 = a.sig * a.sig;
   int si = 0;
   if (GENERAL && a.species) si = a.species[i];
-#ifndef JMD_SPARSE_CHUNK
-#define JMD_SPARSE_CHUNK 4096
-#endif
-#ifndef JMD_SPARSE_TABLE
-#define JMD_SPARSE_TABLE 2048
-#endif
-#ifndef JMD_PAIR_UNROLL
-#define JMD_PAIR_UNROLL 4
-#endif
-  constexpr int UNR = JMD_PAIR_UNROLL;
-  // Interior waves of the Lennard-Jones kernel with scalar parameters gather
-  // through a buffer descriptor of exactly n rows: a padding entry (j = n)
-  // then reads a zero position, so d = -x_i and r^2 >= 3 r_c^2 (every
-  // coordinate of an interior particle is at least r_c), where the switched
-  // or truncated pair term is exactly zero -- no per-pair validity mask and
-  // no index select.  The caller keeps n below 2^27 on this path.
-  constexpr bool kNoMask = INTERIOR && KIND == JMD_LENNARD_JONES && !BOX && !GENERAL &&
-                           DIM == 3 && STRIDE == 4;
-  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(pos), (short)0, (int)(n * 16u), 0x00020000);
-  auto gather = [&](unsigned jraw, float* xj) {
-    if (kNoMask) {
-      const auto v = __builtin_amdgcn_raw_buffer_load_b128(prs, (int)(jraw * 16u), 0, 0);
-      xj[0] = __uint_as_float(v[0]);
-      xj[1] = __uint_as_float(v[1]);
-      xj[2] = __uint_as_float(v[2]);
+  const rsrc_t table = row_table(pos, n, STRIDE * 4);
+  auto gather = [&](unsigned j, float* xj) {
+    if (!INDEXED) {
+      load_pos<DIM, STRIDE>(pos, j < n ? j : i, xj);
+    } else if (DIM == 3) {
+      const f3_t v = struct_load3(table, (int)j, 0, 0, 0);
+      xj[0] = v.x;
+      xj[1] = v.y;
+      xj[2] = v.z;
     } else {
-      load_pos<DIM, STRIDE>(pos, jraw < n ? jraw : i, xj);
+      const f2_t v = struct_load2(table, (int)j, 0, 0, 0);
+      xj[0] = v.x;
+      xj[1] = v.y;
     }
   };
-  // One pair term; padding entries (j = n) read particle i (or, without the
-  // mask, a zero position) and add nothing.
-  auto term = [&](unsigned jraw, const float* xj) {
-    const bool ok = kNoMask || jraw < n;
-    float d[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int c = 0; c < DIM; ++c)
-      d[c] = (INTERIOR || !s.periodic)
-                 ? xj[c] - xi[c]
-                 : min_image_any(xj[c], xi[c], xim[c], s.L[c], s.half[c], s.inbox);
-    if (BOX) box_apply<DIM>(s, d);  // periodic_general: fractional fold, then T
-    float r2 = DIM == 3 ? fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0]))
-                        : fmaf(d[1], d[1], d[0] * d[0]);
+  auto square = [&](const float* d) {
+    return DIM == 3 ? fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0]))
+                    : fmaf(d[1], d[1], d[0] * d[0]);
+  };
+  // One pair term from its difference; masked: `ok` false adds nothing.
+  auto term = [&](unsigned j, const float* d, float r2, bool masked, bool ok) {
     if (GENERAL) {
-      unsigned j = ok ? jraw : i;
       int sj = a.species ? a.species[j] : 0;
       sig = pick(a.sig_mode, a.sig, a.sig_v, i, j, si, sj, a.ns);
       eps = pick(a.eps_mode, a.eps, a.eps_v, i, j, si, sj, a.ns);
-      if (KIND == JMD_SOFT_SPHERE) alp = pick(a.alp_mode, a.alp, a.alp_v, i, j, si, sj, a.ns);
+      if (!LJ) alp = pick(a.alp_mode, a.alp, a.alp_v, i, j, si, sj, a.ns);
     }
-    float dEr;
-    float uu = pair_eval<KIND, SMOOTH>(r2, sig, eps, alp, a, &dEr);
-    dEr = ok ? dEr : 0.0f;
+    float g, u;
+    if (LJ) {
+      g = lj_reduced<SMOOTH>(r2, GENERAL ? sig * sig : sig2, a, &u);
+      if (GENERAL) {
+        g *= eps;
+        if (ENERGY) u *= eps;
+      }
+    } else {
+      u = pair_eval<KIND>(r2, sig, eps, alp, a, &g);
+    }
+    if (masked) g = ok ? g : 0.0f;
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) f[c] = fmaf(dEr, d[c], f[c]);
-    if (ENERGY) *e += ok ? uu : 0.0f;
+    for (int c = 0; c < DIM; ++c) f[c] = fmaf(g, d[c], f[c]);
+    if (ENERGY) *e += masked && !ok ? 0.0f : u;
   };
-  // This lane's entries are sub, sub + TPA, ... < width: nfull blocks of UNR
-  // entries, then fewer than UNR in a tail.  In the blocks every entry lies
-  // in the row, so they are read through one pointer with constant offsets;
-  // the next block's entries are loaded before this block's terms are
-  // computed (software pipeline: one dependent round trip per block, the
-  // position gather).  Rows are left-compacted with padding n, so the row
-  // ends at the first block whose entries are all padding.
-  const int nent = width > sub ? (width - sub + TPA - 1) / TPA : 0;
-  const int nfull = nent / UNR;
-  const int* p = row + sub;
-  if (nfull > 0) {
-    unsigned nxt[UNR];
+  // A block of UNR entries, every one valid in every lane of the wavefront.
+  auto full_block = [&](const unsigned* jj, float (*xj)[3]) {
+    float d[UNR][3];
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) nxt[u] = (unsigned)p[u * TPA];
-    for (int b = 0; b < nfull; ++b) {
-      unsigned jj[UNR];
-      unsigned jmin = n;
+    for (int c = 0; c < DIM; ++c) {
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        jj[u] = nxt[u];
-        jmin = min(jmin, jj[u]);
-      }
-      if (jmin >= n) return;
-      float xj[UNR][3];
+      for (int u = 0; u < UNR; ++u) d[u][c] = xj[u][c] - xi[c];
+      if ((near >> c) & 1u) {
+        float m = 0.0f;  // (a NaN folds to itself, so the maximum may drop it)
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        xj[u][0] = xj[u][1] = xj[u][2] = 0.0f;
-        gather(jj[u], xj[u]);
-      }
-      // next block, clamped to the last full one (re-read, unused, at the end)
-      const int* q = p + min(b + 1, nfull - 1) * (UNR * TPA);
+        for (int u = 0; u < UNR; ++u) m = fmaxf(m, fabsf(d[u][c]));
+        if (__builtin_amdgcn_ballot_w64(m >= s.half[c]) != 0ull) {
+          const float xim = xi[c] - s.L[c];
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) nxt[u] = (unsigned)q[u * TPA];
-      if (__builtin_amdgcn_ballot_w64(jj[UNR - 1] >= n) == 0ull) {
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) term(jj[u], xj[u]);
-      } else {
-        // some row of the wavefront ends in this block: terms only while a
-        // lane still holds an entry (validity is monotone in u per lane)
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-          if (u > 0 && __builtin_amdgcn_ballot_w64(jj[u] < n) == 0ull) break;
-          term(jj[u], xj[u]);
+          for (int u = 0; u < UNR; ++u)
+            d[u][c] = min_image_any(xj[u][c], xi[c], xim, s.L[c], s.half[c], s.inbox);
         }
       }
     }
-  }
-  for (int t = nfull * UNR; t < nent; ++t) {
-    const unsigned j = (unsigned)p[t * TPA];
-    if (j >= n) return;
-    float xj[3] = {0.0f, 0.0f, 0.0f};
-    gather(j, xj);
-    term(j, xj);
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      if (BOX) box_apply<DIM>(s, d[u]);
+      term(jj[u], d[u], square(d[u]), false, true);
+    }
+  };
+  // One entry that is padding in some lane: those add nothing.
+  auto masked_entry = [&](unsigned jraw, const float* xj) {
+    const bool ok = jraw < n;
+    float d[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      d[c] = (near >> c) & 1u
+                 ? min_image_any(xj[c], xi[c], xi[c] - s.L[c], s.L[c], s.half[c], s.inbox)
+                 : xj[c] - xi[c];
+    if (BOX) box_apply<DIM>(s, d);
+    term(ok ? jraw : i, d, square(d), true, ok);
+  };
+  // This lane's entries are sub, sub + TPA, ... < width, in blocks of UNR
+  // (the last one may be short).  The next block's entries are loaded before
+  // this block's terms are computed (software pipeline: one dependent round
+  // trip per block, the position gather).  The row ends at the first block
+  // that is padding in every lane.
+  const unsigned nfull = (unsigned)width / (UNR * TPA);
+  const unsigned nblk = ((unsigned)width + UNR * TPA - 1) / (UNR * TPA);
+  const int* p = row + sub;
+  // (a short block reads its row's last entry where it has none; what it
+  // read is replaced by n when the block is used)
+  auto entries = [&](unsigned b, unsigned* v) {
+    if (b < nfull) {
+      const int* q = p + (long long)b * (UNR * TPA);
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) v[u] = (unsigned)q[u * TPA];
+    } else {
+#pragma unroll
+      for (int u = 0; u < UNR; ++u)
+        v[u] = (unsigned)row[min((int)(b * (UNR * TPA)) + u * TPA + sub, width - 1)];
+    }
+  };
+  unsigned nxt[UNR];
+  if (nblk > 0) entries(0, nxt);
+  for (unsigned b = 0; b < nblk; ++b) {
+    unsigned jj[UNR], jmin = n, jmax = 0u;
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) jj[u] = nxt[u];
+    if (b >= nfull) {
+#pragma unroll
+      for (int u = 0; u < UNR; ++u)
+        if ((int)(b * (UNR * TPA)) + u * TPA + sub >= width) jj[u] = n;
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      jmin = min(jmin, jj[u]);
+      jmax = max(jmax, jj[u]);
+    }
+    if (__builtin_amdgcn_ballot_w64(jmin < n) == 0ull) return;  // the rows have ended
+    float xj[UNR][3];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      xj[u][0] = xj[u][1] = xj[u][2] = 0.0f;
+      gather(jj[u], xj[u]);
+    }
+    // (always issued: a wait that had to allow for both cases would also wait
+    // for these loads)
+    entries(min(b + 1, nblk - 1), nxt);
+    if (__builtin_amdgcn_ballot_w64(jmax >= n) == 0ull) {
+      full_block(jj, xj);
+    } else {
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+        if (__builtin_amdgcn_ballot_w64(jj[u] < n) != 0ull) masked_entry(jj[u], xj[u]);
+      }
+    }
   }
 }
 
@@ -157,14 +220,13 @@ __global__ __launch_bounds__(256) void k_pair_dense(
     half_dt = dt_dev[0] / 2.0f;
   }
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int gt = tile * blockDim.x + threadIdx.x;
-  const int i = gt / TPA;
-  const int sub = gt % TPA;
+  const unsigned gt = (unsigned)tile * 256u + threadIdx.x;
+  const int i = (int)(gt / TPA);
+  const int sub = (int)(gt % TPA);
   const bool active = i < n;
   float f[3] = {0.0f, 0.0f, 0.0f};
   float e = 0.0f;
-  float xi[3] = {0, 0, 0}, xim[3] = {0, 0, 0};
-  bool interior = true;
+  float xi[3] = {0, 0, 0};
   // STEP with TPA >= DIM: lane `sub` of a row's group takes component `sub`
   // of the next step's start; its inputs are loaded here, ahead of the row
   // loop, so their latency hides behind it.
@@ -180,64 +242,60 @@ __global__ __launch_bounds__(256) void k_pair_dense(
     }
     if (kd.gate_next) st_ref = kd.ref[(long long)i * DIM + sub];
   }
+  // (the closing kick without STEP: the row's first lane, loaded ahead too)
+  float pm[3] = {0.0f, 0.0f, 0.0f};
+  if (KICK && !SPREAD && active && sub == 0) {
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) pm[c] = mom[(long long)i * DIM + c];
+  }
   if (active) {
     load_pos<DIM, STRIDE>(pos, i, xi);
+    const int* row = idx + (long long)i * width;
+    unsigned near = 0u;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
-      xim[c] = xi[c] - s.L[c];
-      interior = interior && xi[c] >= a.rc && xi[c] <= s.L[c] - a.rc;
+      // (fractional coordinates: a reach of r_c is r_c |row c of T^-1|)
+      const float w = s.general ? a.rc * s.fw[c] : a.rc;
+      const bool edge = !(s.inbox && xi[c] >= w && xi[c] <= s.L[c] - w);
+      if (s.periodic && __builtin_amdgcn_ballot_w64(edge) != 0ull) near |= 1u << c;
     }
-  }
-  if (s.general && active) {
-    // fractional coordinates: a neighbour within rc of particle i differs by
-    // at most rc |row c of T^-1| in u_c, so no fold is needed when u_c stays
-    // that far from both faces
-    interior = true;
-#pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-      const float w = a.rc * s.fw[c];
-      interior = interior && xi[c] >= w && xi[c] <= 1.0f - w;
-    }
-  }
-  // (n < 2^27 keeps the interior path's buffer offsets j * 16 in range;
-  // the fold-free path is exact only when every neighbour lies in the box)
-  const bool wave_interior =
-      s.inbox && __all(interior || !active) && n < (1 << 27);
-  if (active && s.general) {
-    const int* row = idx + (long long)i * width;
-#define JMD_ROWG(INT, SM)                                                                      \
-  row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, INT, SM, true>(pos, n, s, a, row, width, sub, \
-                                                                  i, xi, xim, f, &e)
-    if (KIND == JMD_LENNARD_JONES && a.smooth) {
-      if (wave_interior) JMD_ROWG(true, 1); else JMD_ROWG(false, 1);
+    // box matrix, switch and table size are uniform: taken once here
+#define JMD_ROW(SM, BX, F32, U)                                                     \
+  row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, SM, BX, F32, U>(pos, n, s, a, row, \
+                                                                   width, sub, i, xi, near, \
+                                                                   f, &e)
+#define JMD_ROW_SM(BX, F32)                                                      \
+  do {                                                                           \
+    if (KIND == JMD_LENNARD_JONES && a.smooth) JMD_ROW(1, BX, F32, 4);           \
+    else JMD_ROW(0, BX, F32, 4);                                                 \
+  } while (0)
+    if ((long long)n * (STRIDE * 4) > 0x7fffffffLL) {
+      // (more than 134 million rows: the compact form)
+      if (s.general) JMD_ROW(-1, true, false, 1);
+      else JMD_ROW(-1, false, false, 1);
+    } else if (s.general) {
+      JMD_ROW_SM(true, true);
     } else {
-      if (wave_interior) JMD_ROWG(true, 0); else JMD_ROWG(false, 0);
+      JMD_ROW_SM(false, true);
     }
-#undef JMD_ROWG
-  } else if (active) {
-    const int* row = idx + (long long)i * width;
-    // the smoothing switch is uniform: taken once here, not per pair
-    if (KIND == JMD_LENNARD_JONES && a.smooth) {
-      if (wave_interior)
-        row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, true, 1>(pos, n, s, a, row, width, sub,
-                                                                  i, xi, xim, f, &e);
-      else
-        row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, false, 1>(pos, n, s, a, row, width, sub,
-                                                                   i, xi, xim, f, &e);
-    } else {
-      if (wave_interior)
-        row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, true, 0>(pos, n, s, a, row, width, sub,
-                                                                  i, xi, xim, f, &e);
-      else
-        row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, false, 0>(pos, n, s, a, row, width, sub,
-                                                                   i, xi, xim, f, &e);
-    }
+#undef JMD_ROW_SM
+#undef JMD_ROW
   }
+  // the Lennard-Jones sums lack -24 epsilon (force) and 4 epsilon (energy)
+  // (lj_reduced), epsilon included per pair where it is not one number
+  constexpr bool LJ = KIND == JMD_LENNARD_JONES;
+  const double eps1 = GENERAL ? 1.0 : (double)a.eps;
   double fd[3];
 #pragma unroll
-  for (int c = 0; c < DIM; ++c) fd[c] = group_sum<TPA>((double)f[c]);
+  for (int c = 0; c < DIM; ++c) {
+    fd[c] = group_sum<TPA>((double)f[c]);
+    if (LJ) fd[c] *= -24.0 * eps1;
+  }
   double ed = 0.0;
-  if (ENERGY) ed = group_sum<TPA>((double)e);
+  if (ENERGY) {
+    ed = group_sum<TPA>((double)e);
+    if (LJ) ed *= 4.0 * eps1;
+  }
   bool moved = false;
   if (SPREAD) {
     // the opening half kick, drift and skin test round every product and
@@ -322,10 +380,10 @@ __global__ __launch_bounds__(256) void k_pair_dense(
     for (int c = 0; c < DIM; ++c) {
       float fc = (float)fd[c];
       if (force) force[(long long)i * DIM + c] = fc;
-      if (KICK && !STEP) mom[(long long)i * DIM + c] = fmaf(half_dt, fc, mom[(long long)i * DIM + c]);
+      if (KICK && !STEP) mom[(long long)i * DIM + c] = fmaf(half_dt, fc, pm[c]);
       if (STEP) {
         fcv[c] = fc;
-        pk[c] = fmaf(half_dt, fc, mom[(long long)i * DIM + c]);
+        pk[c] = fmaf(half_dt, fc, pm[c]);
       }
     }
     if (STEP) {
@@ -403,6 +461,7 @@ void dispatch_dense(int tpa, bool general, const DenseLaunch& L, bool energy, bo
     case 2: JMD_TPA(2); break;
     case 8: JMD_TPA(8); break;
     case 16: JMD_TPA(16); break;
+    case 32: JMD_TPA(32); break;
     default: JMD_TPA(4); break;
   }
 #undef JMD_TPA

@@ -1,0 +1,98 @@
+"""The Dense row kernel at the edges of its blocks: every lane count, row
+widths that end inside and at a block, rows of wavefronts on and off the box
+faces, padding entries in the middle of a row, boxes whose faces are near in
+some dimensions only.  Forces against the float64 sum over the same rows, with
+the bars of test_gpu_pair.py (float32 pair terms: 1e-5 norm-wise, 5e-5 of the
+rms for one particle, 1e-6 for the energy)."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import jaxmd_oracle as O
+from tests.test_gpu_pair import FORCE_RTOL, FORCE_WORST, _force_err
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _rows_fp64(R, sides, idx):
+  """Energy and force of the switched Lennard-Jones rows in float64."""
+  x, L = R.astype(np.float64), np.asarray(sides, np.float64)
+  n = len(x)
+  i, k = np.nonzero(idx < n)
+  d = x[idx[i, k]] - x[i]
+  d -= L * np.rint(d / L)
+  s = (d ** 2).sum(1)
+  c, o = 2.5 ** 2, 2.0 ** 2
+  q6 = s ** -3.0
+  V, dV = 4 * (q6 ** 2 - q6), -24 * (2 * q6 ** 2 - q6) / s
+  S = np.where(s < o, 1.0, (c - s) ** 2 * (c + 2 * s - 3 * o) / (c - o) ** 3)
+  dS = np.where(s < o, 0.0, 12 * (c - s) * (o - s) / (c - o) ** 3)
+  inside = s < c
+  g = np.where(inside, S * dV + dS * V, 0.0)
+  F = np.zeros_like(x)
+  np.add.at(F, i, g[:, None] * d)
+  return 0.5 * np.where(inside, S * V, 0.0).sum(), F
+
+
+def _system(dims, seed):
+  rng = np.random.default_rng(seed)
+  a = (1 / 0.8442) ** (1 / 3)
+  sides = (np.array(dims) * a).astype(np.float32)
+  g = np.stack(np.meshgrid(*[np.arange(d) for d in dims], indexing='ij'), -1).reshape(-1, 3)
+  R = (g + 0.5) * (sides.astype(np.float64) / dims) + rng.normal(0, 0.05, g.shape)
+  R = np.mod(R, sides.astype(np.float64)).astype(np.float32)
+  return np.where(R >= sides, np.float32(0), R), sides
+
+
+@pytest.mark.parametrize('lanes', [0, 2, 4, 8, 16])
+@pytest.mark.parametrize('dims,multiplier,holes', [
+    ((8, 8, 8), 1.0, False),       # all pairs, rows end at their capacity
+    ((9, 8, 14), 1.25, True),      # far faces in one dimension only
+    ((11, 13, 10), 1.0, False),
+    ((16, 9, 9), 1.5, True)])
+def test_rows(lanes, dims, multiplier, holes):
+  import jax_md_amd as jmd
+  R, sides = _system(dims, seed=sum(dims))
+  disp, _ = jmd.space.periodic(sides)
+  nfn, efn = jmd.energy.lennard_jones_neighbor_list(disp, sides, format=jmd.partition.Dense,
+                                                    capacity_multiplier=multiplier)
+  Rt = torch.as_tensor(R, device=DEV)
+  nbrs = nfn.allocate(Rt)
+  if holes:  # a caller that drops pairs by writing N over them
+    rng = np.random.default_rng(1)
+    drop = torch.as_tensor(rng.random(tuple(nbrs.idx.shape)) < 0.1, device=DEV)
+    nbrs.idx[drop] = R.shape[0]
+  E64, F64 = _rows_fp64(R, sides, nbrs.idx.cpu().numpy())
+  lib = jmd._native.load()
+  assert lib.jmd_set_threads_per_atom(lanes) == 0
+  try:
+    for in_box in (False, True):
+      F = efn.force(Rt, nbrs, in_box=in_box)
+      rel, worst = _force_err(F.cpu().numpy(), F64)
+      print(f'rows {dims} lanes {lanes} in_box {in_box}: {rel:.2e} {worst:.2e}', flush=True)
+      assert rel <= FORCE_RTOL and worst <= FORCE_WORST
+    E, _ = efn.energy_and_force(Rt, nbrs)
+    assert abs(float(E) - E64) <= 1e-6 * abs(E64)
+  finally:
+    lib.jmd_set_threads_per_atom(0)
+
+
+@pytest.mark.parametrize('n', [1, 63, 4096, 32184, 70001])
+def test_energy_total_is_the_sum_of_its_rows(n):
+  """The total over block partials against the particles' own energies
+  (float32 each, summed here in float64): 2^-24 of the sum of magnitudes."""
+  import jax_md_amd as jmd
+  g = torch.Generator(device=DEV).manual_seed(n)
+  R = torch.rand((n, 3), generator=g, device=DEV) * 100.0
+  disp, _ = jmd.space.periodic(100.0)
+  nfn, efn = jmd.energy.soft_sphere_neighbor_list(disp, 100.0, sigma=2.0, dr_threshold=0.5,
+                                                  format=jmd.partition.Dense)
+  _, each_fn = jmd.energy.soft_sphere_neighbor_list(disp, 100.0, sigma=2.0, dr_threshold=0.5,
+                                                    per_particle=True,
+                                                    format=jmd.partition.Dense)
+  nbrs = nfn.allocate(R)
+  E, _ = efn.energy_and_force(R, nbrs)
+  each = each_fn(R, nbrs).to(torch.float64)
+  assert abs(float(E) - float(each.sum())) <= 2.0 ** -24 * float(each.abs().sum()) + 1e-30
