@@ -218,6 +218,18 @@ int jmd_remap_neighbor_ids(const int32_t* idx_in, int32_t* idx_out,
                            const int32_t* perm, int64_t n, int32_t format,
                            int64_t width, void* stream);
 
+/* A Sparse-format list from Dense rows [n, width] (padding n or more): each
+ * row's entries in order as (receiver, sender), rows in order (OrderedSparse:
+ * receiver < sender), padding n up to capacity; more entries than that set
+ * JMD_NEIGHBOR_LIST_OVERFLOW in error.  The block loops hand a Sparse-format
+ * list back this way (neighbor formats of jax_md/partition.py:641-661).
+ * workspace: jmd_dense_rows_to_sparse_workspace_bytes(n), 8-byte aligned, no
+ * initial contents. */
+size_t jmd_dense_rows_to_sparse_workspace_bytes(int64_t n);
+int jmd_dense_rows_to_sparse(const int32_t* rows, int64_t n, int64_t width, int32_t format,
+                             int32_t* idx, int64_t capacity, uint8_t* error, void* workspace,
+                             void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Pair reduction                                                            */
 /* ------------------------------------------------------------------------ */

@@ -96,6 +96,9 @@ _SIGNATURES = {
                                    c_int32, c_int32, c_void_p]),
     'jmd_remap_neighbor_ids': (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_int32,
                                          c_int64, c_void_p]),
+    'jmd_dense_rows_to_sparse_workspace_bytes': (c_size_t, [c_int64]),
+    'jmd_dense_rows_to_sparse': (c_int32, [c_void_p, c_int64, c_int64, c_int32, c_void_p, c_int64,
+                                           c_void_p, c_void_p, c_void_p]),
     'jmd_adjoint_workspace_bytes': (c_size_t, [c_int64, c_int32]),
     'jmd_pair_force_vjp': (c_int32, [c_void_p, c_int64, c_int32, c_int32, c_int32,
                                      POINTER(c_float), POINTER(JmdPairPotential), c_void_p,

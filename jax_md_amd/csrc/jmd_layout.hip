@@ -129,6 +129,132 @@ __global__ __launch_bounds__(256) void k_remap_ids(const int* __restrict__ in,
   }
 }
 
+// Dense rows -> a Sparse-format list: each row i's entries j in row order as
+// (receiver j, sender i), rows in order (OrderedSparse: entries below the
+// row's id only), then padding.  Bound by memory: the rows are read twice
+// (once to count, once to write; 36 MB at N = 64,000 stay in the last-level
+// cache between) and the list is written once.  One wavefront per row and 8
+// per workgroup; kRowsPerBlock rows share one partial count, so that the scan
+// between the passes is a single workgroup over n / 64 values.  With torch's
+// masked indexing and cumsum the conversion took 0.75 ms a block at
+// N = 64,000 (it sorted out the kept entries of the flattened rows in several
+// library passes and waited on the host for their number).
+constexpr int kRowsPerBlock = 64;
+
+__device__ __forceinline__ unsigned long long kept_entries(const int* __restrict__ row, int n,
+                                                           int width, int k, int i, int ordered,
+                                                           int* j) {
+  *j = k < width ? row[k] : n;
+  return __builtin_amdgcn_ballot_w64((unsigned)*j < (unsigned)n && (!ordered || *j < i));
+}
+
+constexpr int kSparseBlock = 512;
+
+__global__ __launch_bounds__(kSparseBlock) void k_sparse_count(const int* __restrict__ rows,
+                                                               int n, int width, int ordered,
+                                                               int* __restrict__ row_count,
+                                                               int* __restrict__ block_total) {
+  __shared__ int s_sum[kSparseBlock / kWave];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  int sum = 0;  // wavefront-uniform
+  for (int r = wave; r < kRowsPerBlock; r += kSparseBlock / kWave) {
+    const int i = blockIdx.x * kRowsPerBlock + r;
+    if (i >= n) break;
+    const int* row = rows + (long long)i * width;
+    int count = 0;
+    for (int k = lane; k - lane < width; k += kWave) {
+      int j;
+      count += __popcll(kept_entries(row, n, width, k, i, ordered, &j));
+    }
+    if (lane == 0) row_count[i] = count;
+    sum += count;
+  }
+  if (lane == 0) s_sum[wave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    for (int w = 0; w < kSparseBlock / kWave; ++w) t += s_sum[w];
+    block_total[blockIdx.x] = t;
+  }
+}
+
+// One workgroup: block totals -> exclusive 64-bit offsets, the list's length,
+// and the overflow bit.
+__global__ __launch_bounds__(1024) void k_sparse_offsets(const int* __restrict__ block_total,
+                                                         int nblocks, long long capacity,
+                                                         long long* __restrict__ offset,
+                                                         uint8_t* __restrict__ error) {
+  __shared__ long long s_w[1024 / kWave];
+  const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+  long long carry = 0;
+  for (int b0 = 0; b0 < nblocks; b0 += 1024) {
+    const long long v = b0 + t < nblocks ? block_total[b0 + t] : 0;
+    long long incl = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const long long y = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += y;
+    }
+    if (lane == kWave - 1) s_w[wave] = incl;
+    __syncthreads();
+    long long before = 0, all = 0;
+    for (int w = 0; w < 1024 / kWave; ++w) {
+      before += w < wave ? s_w[w] : 0;
+      all += s_w[w];
+    }
+    if (b0 + t < nblocks) offset[b0 + t] = carry + before + incl - v;
+    carry += all;
+    __syncthreads();  // s_w is rewritten by the next chunk
+  }
+  if (t == 0) {
+    offset[nblocks] = carry;
+    if (carry > capacity) error[0] = (uint8_t)(error[0] | JMD_NEIGHBOR_LIST_OVERFLOW);
+  }
+}
+
+__global__ __launch_bounds__(kSparseBlock) void k_sparse_write(
+    const int* __restrict__ rows, int n, int width, int ordered,
+    const int* __restrict__ row_count, const long long* __restrict__ offset, int nblocks,
+    long long capacity, int* __restrict__ idx) {
+  __shared__ int s_first[kRowsPerBlock];  // a row's first slot inside the block
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  // padding beyond the list's length, spread over the grid
+  for (long long k = offset[nblocks] + (long long)blockIdx.x * kSparseBlock + threadIdx.x;
+       k < capacity; k += (long long)gridDim.x * kSparseBlock) {
+    idx[k] = n;
+    idx[capacity + k] = n;
+  }
+  if (wave == 0) {
+    const int i = blockIdx.x * kRowsPerBlock + lane;
+    const int v = i < n ? row_count[i] : 0;
+    int incl = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int y = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += y;
+    }
+    s_first[lane] = incl - v;
+  }
+  __syncthreads();
+  const long long base = offset[blockIdx.x];
+  for (int r = wave; r < kRowsPerBlock; r += kSparseBlock / kWave) {
+    const int i = blockIdx.x * kRowsPerBlock + r;
+    if (i >= n) break;
+    const int* row = rows + (long long)i * width;
+    long long at = base + s_first[r];
+    for (int k = lane; k - lane < width; k += kWave) {
+      int j;
+      const unsigned long long bal = kept_entries(row, n, width, k, i, ordered, &j);
+      const long long slot = at + wave_prefix_count(bal);
+      if (__builtin_amdgcn_inverse_ballot_w64(bal) && slot < capacity) {
+        idx[slot] = j;             // receiver
+        idx[capacity + slot] = i;  // sender
+      }
+      at += __popcll(bal);
+    }
+  }
+}
+
 static int grid_for(long long total) {
   long long b = (total + 255) / 256;
   if (b < 1) b = 1;
@@ -192,6 +318,39 @@ int jmd_remap_neighbor_ids(const int32_t* idx_in, int32_t* idx_out, const int32_
     hipLaunchKernelGGL(k_remap_ids, dim3(grid_for(width)), dim3(256), 0, st, idx_in, idx_out,
                        perm, (int)n, width, format == JMD_ORDERED_SPARSE ? 1 : 0);
   }
+  JMD_LAUNCH_CHECK();
+  return JMD_OK;
+}
+
+size_t jmd_dense_rows_to_sparse_workspace_bytes(int64_t n) {
+  const long long nb = n > 0 ? (n + kRowsPerBlock - 1) / kRowsPerBlock : 0;
+  return (size_t)(nb + 1) * (sizeof(long long) + sizeof(int)) +
+         (size_t)(n > 0 ? n : 0) * sizeof(int) + 64;
+}
+
+int jmd_dense_rows_to_sparse(const int32_t* rows, int64_t n, int64_t width, int32_t format,
+                             int32_t* idx, int64_t capacity, uint8_t* error, void* workspace,
+                             void* stream) {
+  if (n < 0 || n > 0x7fffffff || width < 0 || width > 0x7fffffff || capacity < 0 ||
+      (format != JMD_SPARSE && format != JMD_ORDERED_SPARSE) || !error || !workspace ||
+      (n > 0 && width > 0 && !rows) || (capacity > 0 && !idx) || ((uintptr_t)workspace & 7) != 0)
+    return JMD_ERR_INVALID;
+  hipStream_t st = (hipStream_t)stream;
+  const int nb = ceil_div(n, kRowsPerBlock);
+  long long* offset = (long long*)workspace;
+  int* total = (int*)(offset + nb + 1);
+  int* row_count = total + nb + 1;
+  const int nn = (int)n, w = (int)width, ordered = format == JMD_ORDERED_SPARSE ? 1 : 0;
+  if (nb > 0) {
+    hipLaunchKernelGGL(k_sparse_count, dim3(nb), dim3(kSparseBlock), 0, st, rows, nn, w, ordered,
+                       row_count, total);
+    JMD_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_sparse_offsets, dim3(1), dim3(1024), 0, st, total, nb, (long long)capacity,
+                     offset, error);
+  JMD_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_sparse_write, dim3(nb > 0 ? nb : 1), dim3(kSparseBlock), 0, st, rows, nn, w,
+                     ordered, row_count, offset, nb, (long long)capacity, idx);
   JMD_LAUNCH_CHECK();
   return JMD_OK;
 }

@@ -282,26 +282,23 @@ def _sparse_to_dense_rows(nbrs, out):
   nbrs.error.code.bitwise_or_(over)
 
 
-def _dense_rows_to_sparse(dense, nbrs):
+def _dense_rows_to_sparse(dense, nbrs, workspace):
   """A Sparse-format list from Dense rows: (receiver j, sender i) for each
   row i's entries in order (OrderedSparse: j < i), rows in order, padded
   with N; more pairs than the list's capacity set the overflow bit."""
-  from . import partition
-  d = dense.idx
-  N = d.shape[0]
-  cap = nbrs.idx.shape[1]
-  keep = d < N
-  if nbrs.format is partition.OrderedSparse:
-    keep = keep & (d < torch.arange(N, device=d.device, dtype=d.dtype)[:, None])
-  flat = keep.reshape(-1)
-  pos = torch.cumsum(flat.to(torch.int64), 0) - 1
-  ok = flat & (pos < cap)
-  senders = torch.arange(N, device=d.device, dtype=torch.int32)[:, None].expand_as(d).reshape(-1)
-  nbrs.idx.fill_(N)
-  nbrs.idx[0, pos[ok]] = d.reshape(-1)[ok]
-  nbrs.idx[1, pos[ok]] = senders[ok]
-  over = (flat.sum() > cap).to(torch.uint8) * int(partition.PEC.NEIGHBOR_LIST_OVERFLOW)
-  nbrs.error.code.bitwise_or_(over)
+  N, width = dense.idx.shape
+  idx = nbrs.idx
+  if idx.dtype != torch.int32 or not idx.is_contiguous():  # a caller's own tensor
+    idx = torch.empty(tuple(idx.shape), dtype=torch.int32, device=idx.device)
+  nat.check(nat.load().jmd_dense_rows_to_sparse(
+      nat.ptr(dense.idx), N, width, nbrs.plan.spec.format_code, nat.ptr(idx), idx.shape[1],
+      nat.ptr(nbrs.error.code), nat.ptr(workspace), nat.stream_handle(idx.device)),
+      'jmd_dense_rows_to_sparse')
+  if idx is not nbrs.idx:
+    nbrs.idx.copy_(idx)
+  # written here, past the tensors' version counters: what other code derived
+  # from the list (its rows, another loop's copies) no longer matches
+  nbrs.plan.epoch += 1
 
 
 class StepEvents:
@@ -400,7 +397,8 @@ class NVELoop:
     # Sparse-format lists run as a Dense copy (deterministic row sums, no
     # float atomics), converted back to the Sparse format after each block
     self.sparse_as_dense = bool(sparse_as_dense)
-    self._shadow = None  # [key, Dense list, Sparse list signature at the last sync]
+    # [key, Dense list, Sparse list signature at the last sync, conversion workspace]
+    self._shadow = None
     self._cont = None  # (signature after the last block, steps since the order was taken)
     # blocks run eagerly (host-launched), graphs recorded, blocks replayed;
     # continued: blocks that started from the previous block's cell order
@@ -539,7 +537,9 @@ class NVELoop:
           cell_list_capacity=nbrs.cell_list_capacity, max_occupancy=width,
           format=partition.Dense, cell_size=nbrs.cell_size, cell_list_fn=None, update_fn=None,
           plan=plan2)
-      self._shadow = [key, shadow, None]
+      back = torch.empty((lib.jmd_dense_rows_to_sparse_workspace_bytes(N),), dtype=torch.uint8,
+                         device=dev)
+      self._shadow = [key, shadow, None, back]
     shadow = self._shadow[1]
     if self._shadow[2] != self._list_signature(nbrs):
       _sparse_to_dense_rows(nbrs, shadow.idx)
@@ -550,7 +550,7 @@ class NVELoop:
     """Writes the block's list back in the Sparse format: each row's entries
     in row order (OrderedSparse: those below the row's id), the reference's
     sender-major layout, overflow when the pairs exceed the capacity."""
-    _dense_rows_to_sparse(shadow, nbrs)
+    _dense_rows_to_sparse(shadow, nbrs, self._shadow[3])
     self._shadow[2] = self._list_signature(nbrs)
     if self._cont is not None:  # the conversion leaves the working copies valid
       self._cont = (self._signature(state, shadow), self._cont[1])
