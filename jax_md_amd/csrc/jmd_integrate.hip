@@ -36,8 +36,7 @@ __global__ __launch_bounds__(256) void k_kick_drift(KickDrift kd, int n) {
     }
   }
   if (kd.gate_next) {
-    const unsigned long long bal = __ballot(moved);
-    if (bal != 0ull && lane_id() == 0) atomicOr(kd.gate_next, 1);
+    raise_gate(kd.gate_next, moved);
   }
 }
 

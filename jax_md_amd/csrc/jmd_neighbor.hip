@@ -881,8 +881,7 @@ __global__ __launch_bounds__(256) void k_bin_slots(const float* __restrict__ pos
     }
   }
   if (kd.active && kd.gate_next) {
-    const unsigned long long bal = __ballot(moved);
-    if (bal != 0ull && lane == 0) atomicOr(kd.gate_next, 1);
+    raise_gate(kd.gate_next, moved);
   }
   if (!open) return;
   // every count was added by the device-scope atomics above
@@ -1167,8 +1166,9 @@ __global__ __launch_bounds__(256) void k_skin_check(const float* __restrict__ po
     load_pos<DIM>(ref, i, b);
     moved = ref_metric_sq<DIM>(a, b, s) > threshold_sq;
   }
-  unsigned long long bal = __ballot(moved);
-  if (bal != 0ull && lane_id() == 0) atomicOr(gate, 1);
+  // one wavefront of the workgroup speaks for all of them
+  moved = __syncthreads_or(moved);
+  if (threadIdx.x < kWave) raise_gate(gate, moved);
 }
 
 // ---------------------------------------------------------------------------

@@ -402,9 +402,7 @@ __global__ __launch_bounds__(256) void k_pair_dense(
     }
   }
   if (ENERGY && active && sub == 0 && e_atom) e_atom[i] = (float)(0.5 * ed);
-  if (STEP && kd.gate_next) {
-    if (__ballot(moved) != 0ull && lane_id() == 0) atomicOr(kd.gate_next, 1);
-  }
+  if (STEP && kd.gate_next) raise_gate(kd.gate_next, moved);
   if (ENERGY) {
     // block partial of 0.5 * sum_i e_i in float64
     __shared__ double s_e[256 / kWave];

@@ -165,8 +165,7 @@ __global__ __launch_bounds__(256) void k_kick_drift64(
     }
   }
   if (gate) {
-    const unsigned long long bal = __ballot(moved);
-    if (bal != 0ull && lane_id() == 0) atomicOr(gate, 1);
+    raise_gate(gate, moved);
   }
 }
 
