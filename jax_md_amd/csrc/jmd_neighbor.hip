@@ -1317,8 +1317,16 @@ static int build_impl(const float* pos, int n, const Space& s, float cutoff_sq,
     A.g = g;
     A.s = s;
     A.cutoff_sq = cutoff_sq;
-    // Bound on |fast d^2 - reference wrapped d^2| in float32: a few roundings
-    // at the scale of 2L on each of the components of d.
+    // Bound on |fast d^2 - reference wrapped d^2| in float32, u = 2^-24, for
+    // positions in [-L, 2L) (others: M_FAR).  Per component the staged image
+    // is off by at most 3 u L (one wrap, one shift), the home position by
+    // u L, their difference rounds by u c; the reference rounds a - b
+    // (3 u L), + L/2 (3.5 u L), + L (u L) and - L/2 (u L / 2): together
+    // 12 u L + u c, so d^2 differs by less than 2 sqrt(3) c (12 u L + u c)
+    // + 7.5 u c^2 < 48 u c (L + c).  A third more covers the box matrix's
+    // products.  Every candidate inside the margin costs two dependent loads
+    // and some 150 operations: with 256 u here a build took 172 us at
+    // N = 262,144, with 64 u it takes 164.
     float Lmax = 0.0f;
     for (int d = 0; d < DIM; ++d) Lmax = fmaxf(Lmax, s.periodic ? s.L[d] : 0.0f);
     if (s.general) {  // real-space extent of the cell: largest row sum of |T|
@@ -1330,7 +1338,7 @@ static int build_impl(const float* pos, int n, const Space& s, float cutoff_sq,
       }
     }
     float c = sqrtf(cutoff_sq);
-    float margin = 128.0f * (c + 1.0f) * (Lmax + c + 1.0f) * 1.1920929e-7f;
+    float margin = 64.0f * (c + 1.0f) * (Lmax + c + 1.0f) * 5.9604645e-8f;
     A.margin = fmaxf(margin, 1e-4f * cutoff_sq);
     A.test = (sparse || ij_rows) ? TEST_IJ : TEST_BOTH;
     A.mask_self = mask_self;
