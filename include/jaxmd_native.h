@@ -430,11 +430,16 @@ typedef struct {
 int jmd_fire_ensemble_max_cells(void);
 
 /* Threads per system workgroup of jmd_fire_ensemble_2d and its adjoint: 256,
- * 512 or 1024; 0 (the default) chooses 1024 when the systems average 4096
- * particles or more, else 512.  A process-wide tuning knob with no
+ * 512 or 1024 for every launch; 0 (the default) leaves it to the launch: the
+ * caller's choice in its mode, else 1024 when the systems average 4096
+ * particles or more and 512 below.  A process-wide tuning knob with no
  * counterpart in the reference; results differ only in the summation order
  * of the workgroup reductions. */
 int jmd_fire_ensemble_set_threads(int32_t threads);
+
+/* The threads per system (512 or 1024) for n_systems systems of n_total
+ * particles, the largest of n_max; no counterpart in the reference. */
+int jmd_fire_ensemble_threads(int32_t n_systems, int64_t n_total, int32_t n_max);
 
 /* Soft-sphere FIRE minimisation of every system of a ragged ensemble, one
  * workgroup per system (systems[order[b]] for workgroup b): the reference's
@@ -448,6 +453,8 @@ int jmd_fire_ensemble_set_threads(int32_t threads);
  *      n_total), F = F(R), P = 0, dt = dt_start, alpha = alpha_start,
  *      energy[s] = E(R)
  *   3  n_steps FIRE steps; energy[s] = E at the end
+ * plus 256 times the threads per system (256, 512 or 1024; 0: chosen by the
+ * systems' average size).
  * fire_params = static_cast float16 values (dt_start, dt_max, n_min, f_inc,
  * f_dec, alpha_start, f_alpha); fire_state [n_systems, 2] = (dt, alpha),
  * fire_n_pos [n_systems]; error [n_systems] sticky overflow bits; builds
@@ -484,7 +491,8 @@ int jmd_fire_ensemble_2d(const jmd_system2d* systems, const int32_t* order, int3
  * step's second node).  mode: 0 initialises x_adjoint = -scale F,
  * p_adjoint = pending = 0, theta = scale dE/dtheta at (position, idx);
  * 1 runs n_steps backward steps through a tape; 2 applies the pending
- * vector at the tape's first node (call once, after the earliest segment).
+ * vector at the tape's first node (call once, after the earliest segment);
+ * plus 256 times the threads per system, as there.
  * box_adjoint (optional, [n_systems] float64): the loss's derivative with
  * respect to each system's box side L, the particles held in real
  * coordinates (the meta-optimisation notebook's periodic_general(L(d) I,

@@ -434,6 +434,7 @@ __device__ __forceinline__ void kick_drift_regs(const KickDrift& kd, long long i
 }
 
 __device__ __forceinline__ int floor_mod_int(int a, int m) {
+  if ((unsigned)a < (unsigned)m) return a;  // its own remainder, without the division
   int r = a % m;
   return r < 0 ? r + m : r;
 }

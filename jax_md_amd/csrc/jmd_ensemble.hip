@@ -20,21 +20,37 @@
 
 namespace jmd {
 
-// Threads per system: 1024 when the systems average 4096 particles or more
-// (16 wavefronts hide the gathers' latency of a large system), else 512
-// (small systems, two workgroups per CU).
+// Threads per system, one workgroup each: 512 keeps two workgroups a CU and
+// wins by 10-35% where every CU has several systems of one size to run (50
+// steps of 512 systems of 512 / 1024 / 2048 particles: 2.4 / 3.4 / 5.3 ms
+// against 3.3 / 3.9 / 5.8); 1024 shortens each system's own chain and wins
+// where the largest one decides (64 systems of 1024 / 2048 / 4000: 1.6 / 2.5 /
+// 4.4 ms against 1.9 / 3.4 / 6.4; 512 systems log-uniform in 64..2048 and
+// 64..4096: 4.0 and 5.4 against 4.4 and 7.4).  So 1024 when the largest system
+// has 768 particles or more (below, its rows leave the second 512 threads too
+// little) and at least a CU's share of all of them; also for an average of
+// 4096, beyond which 512 threads stage no system in LDS.
 constexpr int kEnsThreads = 1024;  // the most a workgroup has
+constexpr int kEnsWaves = 4;       // a SIMD (at 8, 64 VGPRs: the run spilled and took 1.5 times as long)
 static int g_ens_threads = 0;      // jmd_fire_ensemble_set_threads (0: by size)
-inline int ens_threads(int n_systems, long long n_total) {
+constexpr int kEnsCUs = 256;
+inline int ens_threads(int n_systems, long long n_total, long long n_max) {
+  if (n_systems > 0 && n_total / n_systems >= 4096) return 1024;
+  return n_max >= 768 && n_max >= n_total / kEnsCUs ? 1024 : 512;
+}
+// A launch's threads: the override, the caller's (mode >> 8), or the rule for
+// a largest system that is not known (taken as the average).
+inline int ens_launch_threads(int asked, int n_systems, long long n_total) {
   if (g_ens_threads) return g_ens_threads;
+  if (asked) return asked;
   return n_systems > 0 && n_total / n_systems >= 4096 ? 1024 : 512;
 }
+inline bool ens_threads_ok(int threads) {
+  return threads == 0 || threads == 256 || threads == 512 || threads == 1024;
+}
 constexpr int kEnsMaxCells = 8192;
-#ifndef JMD_ENS_ROW_CHUNK
-#define JMD_ENS_ROW_CHUNK 4
-#endif
-constexpr int kEnsRowChunk = JMD_ENS_ROW_CHUNK;  // row entries gathered together (even)
-static_assert(kEnsRowChunk % 2 == 0, "entry parity is the chunk position's");
+constexpr int kEnsBatch = 4;       // elements a streaming pass loads together
+constexpr int kEnsRowChunk = 4;    // row entries gathered together (one 16-byte load)
 constexpr int kEnsParMax = 64;  // species matrices staged in LDS (n_species^2 at most)
 constexpr int kEnsPerThread = 8;  // particles per thread of a system staged in LDS
 static_assert(kEnsThreads * kEnsPerThread <= (1 << 16), "staged ids are 16-bit");
@@ -117,6 +133,17 @@ __device__ __forceinline__ int wg_max(int v, int* s) {
   return r;
 }
 
+// ref_mod64 with the library's fmod out of line: within one period past the
+// box the remainder is the exact difference (L <= x < 2 L), and -L < x < 0 is
+// its own remainder.
+__device__ __noinline__ double ens_mod64_far(double x, double L) { return ref_mod64(x, L); }
+__device__ __forceinline__ double ens_mod64(double x, double L) {
+#pragma clang fp contract(off)
+  if (!(x > -L && x < 2.0 * L)) return ens_mod64_far(x, L);
+  if (x >= L) return x - L;
+  return x < 0.0 ? x + L : x;
+}
+
 // Ascending order of 8 values: Batcher's odd-even merge sort network
 // (19 compare-exchanges, all indices static so the values stay in registers).
 __device__ __forceinline__ void cmp_swap(int& a, int& b) {
@@ -188,13 +215,18 @@ struct EnsView {
 // scatter into sorted[] (system-local), then each cell's ids in ascending
 // order (the stable argsort of partition.py:432).  s_cs holds the counts,
 // then, scanned in place, the starts (cell c spans s_cs[c] .. s_cs[c + 1]).
-// Returns the max filling.
+// Returns the max filling; all_in: every position lies in [0, L].
 template <bool STAGED>
-__device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const EnsView<STAGED>& V,
+__device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const Space& sp,
+                                       const EnsView<STAGED>& V,
                                        int* __restrict__ cellp, int* __restrict__ rankp,
                                        int* __restrict__ sorted, int* s_cs, int* s_red,
-                                       uint16_t* ls) {
+                                       uint16_t* ls, bool* all_in) {
   const int nt = blockDim.x, t = threadIdx.x;
+  bool in = true;  // this thread's positions inside [0, L]
+  auto inside = [&](const float* x) {
+    return x[0] >= 0.0f && x[0] <= sp.L[0] && x[1] >= 0.0f && x[1] <= sp.L[1];
+  };
   for (int c = t; c < g.ncell; c += nt) s_cs[c] = 0;
   __syncthreads();
   // staged system (ls: its cell-sorted ids in LDS): counts here, then after
@@ -205,6 +237,7 @@ __device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const Ens
     for (int a = t; a < S.n; a += nt) {
       float xi[2];
       V.pos(S.offset + a, xi);
+      in = in && inside(xi);
       int ci[2];
       atomicAdd(&s_cs[cell_of<2>(xi, g, ci)], 1);
     }
@@ -212,6 +245,7 @@ __device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const Ens
     for (int a = t; a < S.n; a += nt) {
       float xi[2];
       V.pos(S.offset + a, xi);
+      in = in && inside(xi);
       int ci[2];
       const int h = cell_of<2>(xi, g, ci);
       cellp[a] = h;
@@ -285,8 +319,187 @@ __device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const Ens
   } else {
     for (int c = t; c < g.ncell; c += nt) ens_sort_cell(sorted + s_cs[c], s_cs[c + 1] - s_cs[c]);
   }
-  __syncthreads();
+  *all_in = !__syncthreads_or(!in);
   return wg_max(fill, s_red);
+}
+
+// First slot's rank in a cell's list: slot order is rank (start + k) mod cap,
+// so the first slots hold the members past the next multiple of cap.
+template <bool STAGED>
+__device__ __forceinline__ int ens_first_rank(int start, int m, int cap, float inv_cap) {
+  int over;
+  if constexpr (STAGED) {  // start % cap by the reciprocal, corrected
+    over = start - (int)((float)start * inv_cap) * cap;
+    over = over < 0 ? over + cap : (over >= cap ? over - cap : over);
+  } else {
+    over = start % cap;
+  }
+  const int w = cap - over;
+  return m > w ? w : 0;
+}
+
+// Dense with cells keeps a candidate when both wrap(Ri - Rj) and wrap(Rj - Ri)
+// are inside (partition.py:951,971).
+__device__ __forceinline__ bool ens_exact(const float* xi, const float* xj, const Space& sp,
+                                          float cutoff_sq) {
+  return ref_metric_sq<2>(xi, xj, sp) < cutoff_sq && ref_metric_sq<2>(xj, xi, sp) < cutoff_sq;
+}
+
+// One Dense row as its entries come: rows whose stride is a multiple of 4
+// entries are written 16 bytes at a time (every lane of a store writes a line
+// of its own, so a row costs as many line accesses as it has stores: with
+// 4-byte ones a 4,096-particle build took 14 us longer), entries past the row are counted.
+struct EnsRowOut {
+  int* row;
+  int width, pad, cnt;
+  bool vec;
+  int4 quad;
+  __device__ __forceinline__ EnsRowOut(int* __restrict__ idx, int i, int w, int p)
+      : row(idx + (long long)i * w), width(w), pad(p), cnt(0),
+        vec((w & 3) == 0 && ((uintptr_t)idx & 15) == 0), quad(make_int4(p, p, p, p)) {}
+  __device__ __forceinline__ void put(int j) {
+    if (cnt < width) {
+      if (vec) {
+        const int slot = cnt & 3;
+        quad.x = slot == 0 ? j : quad.x;
+        quad.y = slot == 1 ? j : quad.y;
+        quad.z = slot == 2 ? j : quad.z;
+        quad.w = slot == 3 ? j : quad.w;
+        if (slot == 3) {
+          *reinterpret_cast<int4*>(row + (cnt & ~3)) = quad;
+          quad = make_int4(pad, pad, pad, pad);
+        }
+      } else {
+        row[cnt] = j;
+      }
+    }
+    ++cnt;
+  }
+  __device__ __forceinline__ void close() {  // the open quad, then pads
+    if (vec) {
+      int k = cnt < width ? (cnt & ~3) : width;
+      if (k < width && (cnt & 3) != 0) {
+        *reinterpret_cast<int4*>(row + k) = quad;
+        k += 4;
+      }
+      for (; k < width; k += 4)
+        *reinterpret_cast<int4*>(row + k) = make_int4(pad, pad, pad, pad);
+    } else {
+      for (int k = cnt; k < width; ++k) row[k] = pad;
+    }
+  }
+};
+
+constexpr int kEnsRunMax = 32;  // candidates of three cells in one mask
+
+// Dense rows of a system whose positions all lie in [0, L] and whose cells
+// fit their capacity, three of them a 32-bit mask.  The stencil's cells of one
+// y are consecutive in the sorted ids (two pieces at the box's edge), so a row
+// tests three runs of candidates, four at a time, into three masks, and then
+// emits the kept ones cell by cell in the candidate order (x offset slowest,
+// slots rotated).  Cell by cell, nine short loops took their fullest lane's
+// chunks each and inlined the exact test sixteen times: a 4,096-particle
+// build (1024 threads) took 92 us, this one 59.
+template <bool STAGED>
+__device__ __forceinline__ int ens_rows_runs(const EnsSys& S, const Grid& g, const Space& sp,
+                                             float cutoff_sq, float lo_thr, float hi_thr,
+                                             const EnsView<STAGED>& V,
+                                             const int* __restrict__ sorted, const int* s_cs,
+                                             int* __restrict__ idx, int width, int pad,
+                                             const uint16_t* ls) {
+  const int nt = blockDim.x;
+  const float inv_cap = 1.0f / (float)g.cap;
+  int occ = 0;
+  // rows in cell order: neighbouring lanes read the same candidates
+  for (int s = threadIdx.x; s < S.n; s += nt) {
+    const int a = STAGED ? (int)ls[s] : sorted[s];
+    const int i = S.offset + a;
+    float xi[2];
+    V.pos(i, xi);
+    int ci[2];
+    cell_of<2>(xi, g, ci);  // the binning's cell
+    const int hx = ci[0], hy = ci[1], lx = g.cps[0] - 1, ly = g.cps[1] - 1;
+    const int cx[3] = {hx == 0 ? lx : hx - 1, hx, hx == lx ? 0 : hx + 1};
+    const int cy[3] = {g.cps[0] * (hy == 0 ? ly : hy - 1), g.cps[0] * hy,
+                       g.cps[0] * (hy == ly ? 0 : hy + 1)};
+    unsigned kept[3];
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      const int c0 = cx[0] + cy[y], c1 = cx[1] + cy[y], c2 = cx[2] + cy[y];
+      const int b0 = s_cs[c0], b1 = s_cs[c1], b2 = s_cs[c2];
+      const int m0 = s_cs[c0 + 1] - b0, m01 = m0 + s_cs[c1 + 1] - b1;
+      const int total = m01 + s_cs[c2 + 1] - b2;
+      const int split = hx == 0 ? m0 : m01;
+      const int second = hx == 0 ? b1 - m0 : b2 - m01;
+      unsigned keep = 0, near = 0;
+      for (int f0 = 0; f0 < total; f0 += kEnsRowChunk) {
+        int jl[kEnsRowChunk];
+        float xj[kEnsRowChunk][2];
+#pragma unroll
+        for (int c = 0; c < kEnsRowChunk; ++c) {
+          const int f = min(f0 + c, total - 1);
+          const int at = f + (f < split ? b0 : second);
+          jl[c] = STAGED ? (int)ls[at] : sorted[at];
+        }
+#pragma unroll
+        for (int c = 0; c < kEnsRowChunk; ++c) V.pos(S.offset + jl[c], xj[c]);
+#pragma unroll
+        for (int c = 0; c < kEnsRowChunk; ++c) {
+          // |x_j - x_i| folded: min(|raw|, L - |raw|), positions in the box
+          const float r0 = fabsf(xj[c][0] - xi[0]), r1 = fabsf(xj[c][1] - xi[1]);
+          const float e0 = fminf(r0, sp.L[0] - r0), e1 = fminf(r1, sp.L[1] - r1);
+          const float d2 = fmaf(e1, e1, e0 * e0);
+          const unsigned bit = f0 + c < total && jl[c] != a ? 1u << (f0 + c) : 0u;
+          keep |= d2 < lo_thr ? bit : 0u;
+          near |= d2 <= hi_thr ? bit : 0u;
+        }
+      }
+      near &= ~keep;
+      while (near) {  // within the rounding margin of the cutoff
+        const int f = __ffs((int)near) - 1;
+        near &= near - 1;
+        const int at = f + (f < split ? b0 : second);
+        float xj[2];
+        V.pos(S.offset + (STAGED ? (int)ls[at] : sorted[at]), xj);
+        if (ens_exact(xi, xj, sp, cutoff_sq)) keep |= 1u << f;
+      }
+      kept[y] = keep;
+    }
+    const int cnt = __popc(kept[0]) + __popc(kept[1]) + __popc(kept[2]);
+    occ = max(occ, cnt);
+    if (width > 0) {
+      EnsRowOut out(idx, i, width, pad);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        // the column's kept candidates in slot order, its three cells in turn
+        int start[3], first[3], m[3];
+        unsigned column = 0;
+        int at = 0;
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          const int c = cx[x] + cy[y];
+          start[y] = s_cs[c];
+          m[y] = s_cs[c + 1] - start[y];
+          first[y] = ens_first_rank<STAGED>(start[y], m[y], g.cap, inv_cap);
+          const unsigned bits = kept[y] & ((1u << m[y]) - 1u);
+          kept[y] >>= m[y];  // the run's next cell
+          column |= (bits >> first[y] | (bits & ((1u << first[y]) - 1u)) << (m[y] - first[y])) << at;
+          at += m[y];
+        }
+        while (column) {
+          const int f = __ffs((int)column) - 1;
+          column &= column - 1;
+          const int y1 = f >= m[0], y2 = f >= m[0] + m[1];
+          const int my = y2 ? m[2] : (y1 ? m[1] : m[0]);
+          int k = f - (y2 ? m[0] + m[1] - first[2] : (y1 ? m[0] - first[1] : -first[0]));
+          k = (k >= my ? k - my : k) + (y2 ? start[2] : (y1 ? start[1] : start[0]));
+          out.put(S.offset + (STAGED ? (int)ls[k] : sorted[k]));
+        }
+      }
+      out.close();
+    }
+  }
+  return occ;
 }
 
 // Dense rows of the system (global ids, padding pad) in the reference's
@@ -294,10 +507,9 @@ __device__ __forceinline__ int ens_bin(const EnsSys& S, const Grid& g, const Ens
 template <bool STAGED>
 __device__ __forceinline__ int ens_rows(const EnsSys& S, const Grid& g, const Space& sp,
                                         float cutoff_sq, const EnsView<STAGED>& V,
-                                        const int* __restrict__ cellp,
                         const int* __restrict__ sorted, const int* s_cs,
                         int* __restrict__ idx, int width, int pad, int* s_red,
-                        const uint16_t* ls) {
+                        const uint16_t* ls, bool all_in, int fill) {
   const int nt = blockDim.x, t = threadIdx.x;
   // The candidate test: the minimum-image |x_j - x_i|^2 of positions in the
   // box decides every candidate farther than `margin` from the cutoff (the
@@ -308,95 +520,49 @@ __device__ __forceinline__ int ens_rows(const EnsSys& S, const Grid& g, const Sp
   const float margin =
       fmaxf(128.0f * (rc + 1.0f) * (Lmax + rc + 1.0f) * 1.1920929e-7f, 1e-4f * cutoff_sq);
   const float lo_thr = cutoff_sq - margin, hi_thr = cutoff_sq + margin;
-  // rows whose stride is a multiple of 4 entries are written 16 bytes at a
-  // time: a row's entries collect in a register quad, flushed when full
-  const bool vec = width > 0 && (width & 3) == 0 && ((uintptr_t)idx & 15) == 0;
+  if (all_in && fill <= g.cap && 3 * fill < kEnsRunMax)
+    return wg_max(ens_rows_runs(S, g, sp, cutoff_sq, lo_thr, hi_thr, V, sorted, s_cs, idx, width,
+                                pad, ls),
+                  s_red);
+  const float inv_cap = 1.0f / (float)g.cap;
   int occ = 0;
-  for (int a = t; a < S.n; a += nt) {
+  for (int s = t; s < S.n; s += nt) {
+    const int a = STAGED ? (int)ls[s] : sorted[s];
     const int i = S.offset + a;
     float xi[2];
     V.pos(i, xi);
-    const float xim[2] = {xi[0] - sp.L[0], xi[1] - sp.L[1]};
     const bool in_i = xi[0] >= 0.0f && xi[0] <= sp.L[0] && xi[1] >= 0.0f && xi[1] <= sp.L[1];
     int ci[2];
-    const int h = STAGED ? cell_of<2>(xi, g, ci) : cellp[a];  // the binning's cell
-    const int hx = h % g.cps[0], hy = h / g.cps[0];
+    cell_of<2>(xi, g, ci);  // the binning's cell
+    const int hx = ci[0], hy = ci[1];
     // the stencil's columns and rows, wrapped by comparison (offsets of one)
     const int cx[3] = {hx == 0 ? g.cps[0] - 1 : hx - 1, hx, hx + 1 == g.cps[0] ? 0 : hx + 1};
     const int cy[3] = {hy == 0 ? g.cps[1] - 1 : hy - 1, hy, hy + 1 == g.cps[1] ? 0 : hy + 1};
-    int cnt = 0;
-    int4 quad = make_int4(pad, pad, pad, pad);
-    int* row = idx + (long long)i * width;
+    EnsRowOut out(idx, i, width, pad);
     for (int st = 0; st < 9; ++st) {  // iota order, x offset slowest
       const int c = cx[st / 3] + g.cps[0] * cy[st % 3];
       const int start = s_cs[c];
       const int m = min(s_cs[c + 1] - start, g.cap);
-      const int w = g.cap - (start % g.cap);
-      // the cell's members in chunks: ids, then their positions, then the
-      // tests in slot order
-      for (int q0 = 0; q0 < m; q0 += kEnsRowChunk) {
-        int jl[kEnsRowChunk];
-        float xj[kEnsRowChunk][2];
-#pragma unroll
-        for (int c2 = 0; c2 < kEnsRowChunk; ++c2) {
-          const int q = q0 + c2;
-          int k = q;  // slot order: rank (start + k) mod cap
-          if (m > w) k = (q < m - w) ? (w + q) : (q - (m - w));
-          jl[c2] = q < m ? (STAGED ? (int)ls[start + k] : sorted[start + k]) : -1;
-        }
-#pragma unroll
-        for (int c2 = 0; c2 < kEnsRowChunk; ++c2) {
-          xj[c2][0] = xj[c2][1] = 0.0f;
-          if (jl[c2] >= 0) V.pos(S.offset + jl[c2], xj[c2]);
-        }
-#pragma unroll
-        for (int c2 = 0; c2 < kEnsRowChunk; ++c2) {
-          if (jl[c2] < 0 || jl[c2] == a) continue;  // past the cell; mask_self
-          const int j = S.offset + jl[c2];
-          const float e0 = min_image_disp(xj[c2][0], xi[0], xim[0], sp.L[0], sp.half[0]);
-          const float e1 = min_image_disp(xj[c2][1], xi[1], xim[1], sp.L[1], sp.half[1]);
-          const float d2 = fmaf(e1, e1, e0 * e0);
-          const bool in_j = xj[c2][0] >= 0.0f && xj[c2][0] <= sp.L[0] && xj[c2][1] >= 0.0f &&
-                            xj[c2][1] <= sp.L[1];
-          bool keep = in_i && in_j && d2 < lo_thr;
-          // Dense with cells keeps a candidate when both wrap(Ri - Rj) and
-          // wrap(Rj - Ri) are inside (partition.py:951,971)
-          if (!keep && (!(in_i && in_j) || d2 <= hi_thr))
-            keep = ref_metric_sq<2>(xi, xj[c2], sp) < cutoff_sq &&
-                   ref_metric_sq<2>(xj[c2], xi, sp) < cutoff_sq;
-          if (keep) {
-            if (cnt < width) {
-              if (vec) {
-                const int slot = cnt & 3;
-                quad.x = slot == 0 ? j : quad.x;
-                quad.y = slot == 1 ? j : quad.y;
-                quad.z = slot == 2 ? j : quad.z;
-                quad.w = slot == 3 ? j : quad.w;
-                if (slot == 3) {
-                  *reinterpret_cast<int4*>(row + (cnt & ~3)) = quad;
-                  quad = make_int4(pad, pad, pad, pad);
-                }
-              } else {
-                row[cnt] = j;
-              }
-            }
-            ++cnt;
-          }
-        }
+      const int k_first = ens_first_rank<STAGED>(start, m, g.cap, inv_cap);
+      for (int q = 0; q < m; ++q) {  // slot order
+        int k = q + k_first;
+        k = k >= m ? k - m : k;
+        const int jl = STAGED ? (int)ls[start + k] : sorted[start + k];
+        if (jl == a) continue;  // mask_self
+        float xj[2];
+        V.pos(S.offset + jl, xj);
+        const float r0 = fabsf(xj[0] - xi[0]), r1 = fabsf(xj[1] - xi[1]);
+        const float e0 = fminf(r0, sp.L[0] - r0), e1 = fminf(r1, sp.L[1] - r1);
+        const float d2 = fmaf(e1, e1, e0 * e0);
+        const bool in = in_i && xj[0] >= 0.0f && xj[0] <= sp.L[0] && xj[1] >= 0.0f &&
+                        xj[1] <= sp.L[1];
+        bool keep = in && d2 < lo_thr;
+        if (!keep && (!in || d2 <= hi_thr)) keep = ens_exact(xi, xj, sp, cutoff_sq);
+        if (keep) out.put(S.offset + jl);
       }
     }
-    if (vec) {
-      // the partial quad (pads after the last entry), then whole pad quads
-      int k = cnt < width ? (cnt & ~3) : width;
-      if (k < width && (cnt & 3) != 0) {
-        *reinterpret_cast<int4*>(row + k) = quad;
-        k += 4;
-      }
-      for (; k < width; k += 4) *reinterpret_cast<int4*>(row + k) = make_int4(pad, pad, pad, pad);
-    } else {
-      for (int k = cnt; k < width; ++k) row[k] = pad;
-    }
-    occ = max(occ, cnt);
+    out.close();
+    occ = max(occ, out.cnt);
   }
   return wg_max(occ, s_red);
 }
@@ -422,14 +588,28 @@ __device__ __forceinline__ const float* ens_stage_params(const PairArgs& a,
 }
 
 // sigma, epsilon, alpha (which = 0, 1, 2) of pair (i, j), species matrices
-// from LDS when staged.
+// from LDS when staged.  PLAIN (ens_plain): epsilon scalar, alpha = 2, sigma
+// scalar or staged; the row loops then hold no power function and no gathers
+// of parameters (with them inlined four times a chunk the run kernel was
+// 94 KB of code and spilled at 128 VGPRs).
+template <bool PLAIN>
 __device__ __forceinline__ float ens_pick(const PairArgs& a, int which, const float* par, int i,
                                           int j, int si, int sj) {
+  if constexpr (PLAIN) {
+    if (which == 0) return a.sig_mode == JMD_PARAM_SPECIES ? par[si * a.ns + sj] : a.sig;
+    return which == 1 ? a.eps : 2.0f;
+  }
   const int mode = which == 0 ? a.sig_mode : (which == 1 ? a.eps_mode : a.alp_mode);
   if (par && mode == JMD_PARAM_SPECIES) return par[which * kEnsParMax + si * a.ns + sj];
   return which == 0 ? pick(a.sig_mode, a.sig, a.sig_v, i, j, si, sj, a.ns)
                     : (which == 1 ? pick(a.eps_mode, a.eps, a.eps_v, i, j, si, sj, a.ns)
                                   : pick(a.alp_mode, a.alp, a.alp_v, i, j, si, sj, a.ns));
+}
+
+inline bool ens_plain(const PairArgs& a) {
+  return a.eps_mode == JMD_PARAM_SCALAR && a.alp_mode == JMD_PARAM_SCALAR && a.alp == 2.0f &&
+         (a.sig_mode == JMD_PARAM_SCALAR ||
+          (a.sig_mode == JMD_PARAM_SPECIES && a.ns >= 1 && a.ns * a.ns <= kEnsParMax));
 }
 
 // dsig[si, sj], from LDS when staged.
@@ -438,14 +618,38 @@ __device__ __forceinline__ float ens_dsig(const PairArgs& a, const float* __rest
   return par ? par[3 * kEnsParMax + si * a.ns + sj] : dsig[si * a.ns + sj];
 }
 
+// One Dense row read kEnsRowChunk entries at a time: a 16-byte load where the
+// row stride is a multiple of 4 entries, else single loads; pads past its end.
+struct EnsRow {
+  const int* row;
+  int width, pad;
+  bool vec;
+  __device__ __forceinline__ EnsRow(const int* __restrict__ idx, int i, int w, int p)
+      : row(idx + (long long)i * w), width(w), pad(p),
+        vec((w & 3) == 0 && ((uintptr_t)idx & 15) == 0) {}
+  __device__ __forceinline__ int4 chunk(int k) const {
+    int4 q = make_int4(pad, pad, pad, pad);
+    if (vec) {
+      if (k < width) q = *reinterpret_cast<const int4*>(row + k);
+    } else {
+      if (k < width) q.x = row[k];
+      if (k + 1 < width) q.y = row[k + 1];
+      if (k + 2 < width) q.z = row[k + 2];
+      if (k + 3 < width) q.w = row[k + 3];
+    }
+    return q;
+  }
+};
+
 // Soft-sphere force of row i: two accumulators (entries k even / odd) summed
 // in float64, as the Dense kernel's two lanes per row do; optional energy.
-template <bool STAGED>
+template <bool STAGED, bool PLAIN>
 __device__ __forceinline__ void ens_force_row(int i, const EnsView<STAGED>& V,
                                               const int* __restrict__ idx, int width, int pad,
                                               const Space& sp, const PairArgs& a,
                                               const float* par, float* F, double* e) {
 #pragma clang fp contract(off)
+  const EnsRow R(idx, i, width, pad);
   float xi[2], xim[2];
   V.pos(i, xi);
   xim[0] = xi[0] - sp.L[0];
@@ -453,24 +657,15 @@ __device__ __forceinline__ void ens_force_row(int i, const EnsView<STAGED>& V,
   float f[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
   float en[2] = {0.0f, 0.0f};
   const int si = V.species(i);
-  const int* row = idx + (long long)i * width;
   // The row in chunks: the chunk's ids, then all its gathers (position,
   // species), then the terms in entry order; a row ends at its first pad.
-  // rows whose stride is a multiple of 4 entries are read 16 bytes at a time
-  const bool vec = kEnsRowChunk == 4 && (width & 3) == 0 && ((uintptr_t)idx & 15) == 0;
+  int4 ids = R.chunk(0), next = R.chunk(kEnsRowChunk);
   for (int k0 = 0; k0 < width; k0 += kEnsRowChunk) {
-    int js[kEnsRowChunk], sjs[kEnsRowChunk];
+    const int js[kEnsRowChunk] = {ids.x, ids.y, ids.z, ids.w};
+    ids = next;
+    next = R.chunk(k0 + 2 * kEnsRowChunk);
+    int sjs[kEnsRowChunk];
     float xj[kEnsRowChunk][2];
-    if (vec) {
-      const int4 q = *reinterpret_cast<const int4*>(row + k0);
-      js[0] = q.x;
-      js[1 % kEnsRowChunk] = q.y;
-      js[2 % kEnsRowChunk] = q.z;
-      js[3 % kEnsRowChunk] = q.w;
-    } else {
-#pragma unroll
-      for (int c = 0; c < kEnsRowChunk; ++c) js[c] = k0 + c < width ? row[k0 + c] : pad;
-    }
 #pragma unroll
     for (int c = 0; c < kEnsRowChunk; ++c) {
       xj[c][0] = xj[c][1] = 0.0f;
@@ -493,9 +688,9 @@ __device__ __forceinline__ void ens_force_row(int i, const EnsView<STAGED>& V,
       d[1] = min_image_disp(xj[c][1], xi[1], xim[1], sp.L[1], sp.half[1]);
       const float r2 = fmaf(d[1], d[1], d[0] * d[0]);
       const int sj = sjs[c];
-      const float sig = ens_pick(a, 0, par, i, j, si, sj);
-      const float eps = ens_pick(a, 1, par, i, j, si, sj);
-      const float alp = ens_pick(a, 2, par, i, j, si, sj);
+      const float sig = ens_pick<PLAIN>(a, 0, par, i, j, si, sj);
+      const float eps = ens_pick<PLAIN>(a, 1, par, i, j, si, sj);
+      const float alp = ens_pick<PLAIN>(a, 2, par, i, j, si, sj);
       float dEr;
       const float u = pair_eval<JMD_SOFT_SPHERE>(r2, sig, eps, alp, a, &dEr);
       const int l = c & 1;  // k0 is even: the parity of k = k0 + c
@@ -510,10 +705,26 @@ __device__ __forceinline__ void ens_force_row(int i, const EnsView<STAGED>& V,
   if (e) *e += 0.5 * ((double)en[0] + (double)en[1]);
 }
 
+// Copies a system's rows between two Dense lists of one width, 16 bytes at a
+// time where the rows allow it.
+__device__ __forceinline__ void ens_copy_rows(const EnsSys& S, int* __restrict__ to,
+                                              const int* __restrict__ from, int width) {
+  const long long base = (long long)S.offset * width, rows = (long long)S.n * width;
+  if ((width & 3) == 0 && (((uintptr_t)to | (uintptr_t)from) & 15) == 0) {
+    const int4* src = reinterpret_cast<const int4*>(from + base);
+    int4* dst = reinterpret_cast<int4*>(to + base);
+#pragma unroll 4
+    for (long long q = threadIdx.x; q < rows / 4; q += blockDim.x) dst[q] = src[q];
+  } else {
+#pragma unroll 4
+    for (long long q = threadIdx.x; q < rows; q += blockDim.x) to[base + q] = from[base + q];
+  }
+}
+
 // STAGED: the systems of at most lds_n particles, kept in LDS; else the
 // larger ones, read from global memory.  Each instance skips the other's.
-template <bool STAGED>
-__global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
+template <bool STAGED, bool PLAIN, bool RUN>
+__global__ __launch_bounds__(kEnsThreads, kEnsWaves) void k_fire_ensemble(
     const EnsSys* __restrict__ systems, const int* __restrict__ order, int nsys, int ntot,
     int mode, int n_steps, double* __restrict__ x_hi, float* __restrict__ x,
     float* __restrict__ p, float* __restrict__ F, float* __restrict__ x_ref,
@@ -578,25 +789,29 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
   g.cap = S.cap;
   const int pad = ntot;
 
-  if (mode == ENS_FILL) {
+  if (!RUN && mode == ENS_FILL) {
     Grid g2 = g;
     g2.cps[0] = S.fill_cps[0];
     g2.cps[1] = S.fill_cps[1];
     g2.cell_size[0] = S.fill_cell_size[0];
     g2.cell_size[1] = S.fill_cell_size[1];
     g2.ncell = g2.cps[0] * g2.cps[1];
-    const int fill = ens_bin(S, g2, V, cellp, rankp, sorted, s_cs, s_red, lsorted);
+    bool all_in;
+    const int fill = ens_bin(S, g2, sp, V, cellp, rankp, sorted, s_cs, s_red, lsorted, &all_in);
     if (t == 0) out_stat[sid] = fill;
     return;
   }
 
   uint8_t err = 0;
   int nbuilds = 0;
+  int* list = idx;    // the rows a rebuild writes and the forces read
+  int list_slot = 0;  // its tape slot (record_node(0) fills 0)
   // list build at the current positions (allocate / update)
   auto rebuild = [&](bool store) {
-    const int fill = ens_bin(S, g, V, cellp, rankp, sorted, s_cs, s_red, lsorted);
-    const int occ = ens_rows(S, g, sp, cutoff_sq, V, cellp, sorted, s_cs, idx,
-                             store ? width : 0, pad, s_red, lsorted);
+    bool all_in;
+    const int fill = ens_bin(S, g, sp, V, cellp, rankp, sorted, s_cs, s_red, lsorted, &all_in);
+    const int occ = ens_rows(S, g, sp, cutoff_sq, V, sorted, s_cs, list,
+                             store ? width : 0, pad, s_red, lsorted, all_in, fill);
     if (fill > g.cap) err |= JMD_CELL_LIST_OVERFLOW;
     if (occ > S.max_occ) err |= JMD_NEIGHBOR_LIST_OVERFLOW;
     for (int q = t; q < S.n; q += nt) {
@@ -608,21 +823,21 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
     return occ;
   };
 
-  if (mode == ENS_OCCUPANCY) {
+  if (!RUN && mode == ENS_OCCUPANCY) {
     const int occ = rebuild(false);
     if (t == 0) out_stat[sid] = occ;
     return;
   }
 
   const double L0 = S.side[0], L1 = S.side[1];
-  if (mode == ENS_INIT) {
+  if (!RUN) {  // ENS_INIT
     rebuild(true);
     __syncthreads();
     double e = 0.0, z1 = 0.0, z2 = 0.0;
     for (int q = t; q < S.n; q += nt) {
       const int i = S.offset + q;
       float f[2];
-      ens_force_row(i, V, idx, width, pad, sp, a, par, f, &e);
+      ens_force_row<STAGED, PLAIN>(i, V, idx, width, pad, sp, a, par, f, &e);
       F[2LL * i] = f[0];
       F[2LL * i + 1] = f[1];
       p[2LL * i] = 0.0f;
@@ -655,12 +870,12 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
       tape.x[k * n2 + g] = x[g];
       tape.F[k * n2 + g] = F[g];
     }
-    const long long rows = (long long)S.n * width;
-    int* dst = tape.idx + (long long)k * ntot * width + (long long)S.offset * width;
-    const int* src = idx + (long long)S.offset * width;
-    for (long long q = t; q < rows; q += nt) dst[q] = src[q];
+    ens_copy_rows(S, tape.idx + (long long)k * ntot * width, idx, width);
   };
   if (tape.x) record_node(0);
+  // a taped segment keeps its current list in the tape's slot (a rebuild then
+  // writes the next slot and nothing is copied); idx gets the last one at the
+  // end
   // The half-step pass also makes the next step's skin test (on the
   // positions it writes, against the reference positions, which only a
   // rebuild changes, before the half-step) and applies the previous step's
@@ -670,7 +885,6 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
   // the pending mixing's ratio, keep and alpha (workgroup-uniform: in LDS,
   // out of the registers the force loop needs)
   __shared__ double s_mix[3];
-  int list_slot = 0;  // tape slot of the current list (record_node(0) fills 0)
   bool moved_next = false;
   bool mix_pending = false;
   for (int step = 0; step < n_steps; ++step) {
@@ -686,15 +900,14 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
       }
     }
     const bool rebuilt = __syncthreads_or(moved);
-    if (rebuilt) rebuild(true);
-    __syncthreads();
-    if (tape.x && rebuilt) {  // the list the force at node step + 1 will use
-      list_slot = step + 1;
-      const long long rows = (long long)S.n * width;
-      int* dst = tape.idx + (long long)(step + 1) * ntot * width + (long long)S.offset * width;
-      const int* src = idx + (long long)S.offset * width;
-      for (long long q = t; q < rows; q += nt) dst[q] = src[q];
+    if (rebuilt) {
+      if (tape.x) {  // the list the force at node step + 1 will use
+        list_slot = step + 1;
+        list = tape.idx + (long long)list_slot * ntot * width;
+      }
+      rebuild(true);
     }
+    __syncthreads();
     // velocity-Verlet sub-step at the FIRE time step (float16 value), one
     // particle per iteration
     const float dt = s_scal[0];
@@ -702,65 +915,77 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
     const double mix_ratio = s_mix[0], mix_keep = s_mix[1];
     const float mix_alpha = (float)s_mix[2];
     moved_next = false;
-    for (int q = t; q < S.n; q += nt) {
-      const long long g0 = 2LL * (S.offset + q);
-      float xn[2];
+    // two particles at a time, all their loads before any store
+    for (int q0 = t; q0 < S.n; q0 += 2 * nt) {
+      float pq[2][2], fq[2][2], ri[2][2];
+      double xq[2][2];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const long long gq = g0 + c;
-        float p0 = p[gq];
-        const float fq = F[gq];
-        if (mix_pending) {  // the previous step's FIRE mixing
-          double pv = p0;
-          pv = pv + (double)mix_alpha * ((double)fq * mix_ratio - pv);
-          p0 = (float)(pv * mix_keep);
+      for (int u = 0; u < 2; ++u) {
+        const int q = min(q0 + u * nt, S.n - 1);
+        const long long g0 = 2LL * (S.offset + q);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          pq[u][c] = p[g0 + c];
+          fq[u][c] = F[g0 + c];
+          xq[u][c] = x_hi[g0 + c];
         }
-        const float pk = p0 + half * fq;
-        double xv = x_hi[gq] + (double)dt * (double)pk;
-        xv = ref_mod64(xv, c ? L1 : L0);
-        p[gq] = pk;
-        x_hi[gq] = xv;
-        xn[c] = (float)xv;
-        x[gq] = xn[c];
-        if constexpr (STAGED) lx[2 * q + c] = xn[c];
+        load_pos<2>(x_ref, S.offset + q, ri[u]);
       }
-      float ri[2];
-      load_pos<2>(x_ref, S.offset + q, ri);
-      moved_next = moved_next || ref_metric_sq<2>(xn, ri, sp) > thr_sq;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int q = q0 + u * nt;
+        if (q >= S.n) break;
+        const long long g0 = 2LL * (S.offset + q);
+        float xn[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const long long gq = g0 + c;
+          float p0 = pq[u][c];
+          if (mix_pending) {  // the previous step's FIRE mixing
+            double pv = p0;
+            pv = pv + (double)mix_alpha * ((double)fq[u][c] * mix_ratio - pv);
+            p0 = (float)(pv * mix_keep);
+          }
+          const float pk = p0 + half * fq[u][c];
+          double xv = xq[u][c] + (double)dt * (double)pk;
+          xv = ens_mod64(xv, c ? L1 : L0);
+          p[gq] = pk;
+          x_hi[gq] = xv;
+          xn[c] = (float)xv;
+          x[gq] = xn[c];
+          if constexpr (STAGED) lx[2 * q + c] = xn[c];
+        }
+        moved_next = moved_next || ref_metric_sq<2>(xn, ri[u], sp) > thr_sq;
+      }
     }
     __syncthreads();
+    // forces of the new positions, the second half kick and the FIRE sums
+    double ff = 0.0, pp = 0.0, fp = 0.0;
     for (int q = t; q < S.n; q += nt) {
       const int i = S.offset + q;
-      float f[2];
-      ens_force_row(i, V, idx, width, pad, sp, a, par, f, nullptr);
-      F[2LL * i] = f[0];
-      F[2LL * i + 1] = f[1];
-    }
-    __syncthreads();
-    double ff = 0.0, pp = 0.0, fp = 0.0;
-    if (tape.x) {
-      for (int k = t; k < 2 * S.n; k += nt) {
-        const long long q = 2LL * S.offset + k;
-        const float pk = p[q] + half * F[q];
-        p[q] = pk;
-        const double fv = F[q], pv = pk;
+      float pk[2], f[2];
+      load_pos<2>(p, i, pk);
+      ens_force_row<STAGED, PLAIN>(i, V, list, width, pad, sp, a, par, f, nullptr);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        pk[c] = pk[c] + half * f[c];
+        const double fv = f[c], pv = pk[c];
         ff += fv * fv;
         pp += pv * pv;
         fp += fv * pv;
-        tape.q[step * n2 + q] = pk;
-        tape.x[(step + 1) * n2 + q] = x[q];
-        tape.F[(step + 1) * n2 + q] = F[q];
       }
-    } else {
-#pragma unroll 4
-      for (int k = t; k < 2 * S.n; k += nt) {
-        const long long q = 2LL * S.offset + k;
-        const float pk = p[q] + half * F[q];
-        p[q] = pk;
-        const double fv = F[q], pv = pk;
-        ff += fv * fv;
-        pp += pv * pv;
-        fp += fv * pv;
+      store_pos<2>(F, i, f);
+      store_pos<2>(p, i, pk);
+      if (tape.x) {
+        const long long g0 = 2LL * i;
+        float xi[2];
+        V.pos(i, xi);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          tape.q[step * n2 + g0 + c] = pk[c];
+          tape.x[(step + 1) * n2 + g0 + c] = xi[c];
+          tape.F[(step + 1) * n2 + g0 + c] = f[c];
+        }
       }
     }
     wg_sum3(ff, pp, fp, s_d);
@@ -809,8 +1034,9 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble(
   double e = 0.0, z1 = 0.0, z2 = 0.0;
   for (int q = t; q < S.n; q += nt) {
     float f[2];
-    ens_force_row(S.offset + q, V, idx, width, pad, sp, a, par, f, &e);
+    ens_force_row<STAGED, PLAIN>(S.offset + q, V, list, width, pad, sp, a, par, f, &e);
   }
+  if (list != idx) ens_copy_rows(S, idx, list, width);
   wg_sum3(e, z1, z2, s_d);
   if (t == 0) {
     fire_state[2 * sid] = s_scal[0];
@@ -861,7 +1087,7 @@ __device__ __forceinline__ float image_of(float raw, float half) {
 // h_i = (J v)_i over the system's rows at positions x with list idx; returns
 // this thread's share of v^T dF/dtheta (rows it owns) and, with box, adds its
 // share of v^T dF/dL to lacc.
-template <bool STAGED>
+template <bool STAGED, bool PLAIN>
 __device__ __forceinline__ double ens_hvp_rows(const EnsSys& S, const Space& sp,
                                                const PairArgs& a, const float* par,
                                                const float* __restrict__ dsig,
@@ -872,8 +1098,6 @@ __device__ __forceinline__ double ens_hvp_rows(const EnsSys& S, const Space& sp,
                                                double& lacc) {
 #pragma clang fp contract(off)
   double tacc = 0.0;
-  // rows whose stride is a multiple of 4 entries are read 16 bytes at a time
-  const bool vec = kEnsRowChunk == 4 && (width & 3) == 0 && ((uintptr_t)idx & 15) == 0;
   for (int q = threadIdx.x; q < S.n; q += blockDim.x) {
     const int i = S.offset + q;
     float xi[2], xim[2], vi[2];
@@ -883,21 +1107,15 @@ __device__ __forceinline__ double ens_hvp_rows(const EnsSys& S, const Space& sp,
     xim[1] = xi[1] - sp.L[1];
     const int si = XV.species(i);
     float h0 = 0.0f, h1 = 0.0f, tp = 0.0f, lp = 0.0f;
-    const int* row = idx + (long long)i * width;
+    const EnsRow R(idx, i, width, pad);
+    int4 ids = R.chunk(0), next = R.chunk(kEnsRowChunk);
     // the row in chunks: ids, then their gathers, then the terms in order
     for (int k0 = 0; k0 < width; k0 += kEnsRowChunk) {
-      int js[kEnsRowChunk], sjs[kEnsRowChunk];
+      const int js[kEnsRowChunk] = {ids.x, ids.y, ids.z, ids.w};
+      ids = next;
+      next = R.chunk(k0 + 2 * kEnsRowChunk);
+      int sjs[kEnsRowChunk];
       float xj[kEnsRowChunk][2], vj[kEnsRowChunk][2];
-      if (vec) {
-        const int4 q4 = *reinterpret_cast<const int4*>(row + k0);
-        js[0] = q4.x;
-        js[1 % kEnsRowChunk] = q4.y;
-        js[2 % kEnsRowChunk] = q4.z;
-        js[3 % kEnsRowChunk] = q4.w;
-      } else {
-#pragma unroll
-        for (int c = 0; c < kEnsRowChunk; ++c) js[c] = k0 + c < width ? row[k0 + c] : pad;
-      }
 #pragma unroll
       for (int c = 0; c < kEnsRowChunk; ++c) {
         xj[c][0] = xj[c][1] = vj[c][0] = vj[c][1] = 0.0f;
@@ -923,9 +1141,9 @@ __device__ __forceinline__ double ens_hvp_rows(const EnsSys& S, const Space& sp,
         w[1] = vj[c][1] - vi[1];
         const float r2 = fmaf(d[1], d[1], d[0] * d[0]);
         const int sj = sjs[c];
-        const float sig = ens_pick(a, 0, par, i, j, si, sj);
-        const float eps = ens_pick(a, 1, par, i, j, si, sj);
-        const float alp = ens_pick(a, 2, par, i, j, si, sj);
+        const float sig = ens_pick<PLAIN>(a, 0, par, i, j, si, sj);
+        const float eps = ens_pick<PLAIN>(a, 1, par, i, j, si, sj);
+        const float alp = ens_pick<PLAIN>(a, 2, par, i, j, si, sj);
         const PairD2 D = pair_eval2<JMD_SOFT_SPHERE>(r2, sig, eps, alp, a);
         const float dw = fmaf(d[1], w[1], d[0] * w[0]);
         const float tt = 2.0f * D.gp * dw;
@@ -958,8 +1176,8 @@ __device__ __forceinline__ double ens_hvp_rows(const EnsSys& S, const Space& sp,
 // STAGED: systems of at most lds_n particles, with the positions of the
 // node and the vector of each Jacobian product copied to LDS; else the
 // larger ones, read from memory.  Each instance skips the other's systems.
-template <bool STAGED>
-__global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble_back(
+template <bool STAGED, bool PLAIN>
+__global__ __launch_bounds__(kEnsThreads, kEnsWaves) void k_fire_ensemble_back(
     const EnsSys* __restrict__ systems, int nsys, int ntot, int mode, int K,
     const float* __restrict__ x, const float* __restrict__ F, const int* __restrict__ idx,
     int width, PairArgs a0, const float* __restrict__ dsig0, EnsTape tape,
@@ -1027,9 +1245,9 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble_back(
           d[1] = min_image_disp(xj[1], xi[1], xim[1], sp.L[1], sp.half[1]);
           const float r2 = fmaf(d[1], d[1], d[0] * d[0]);
           const int sj = a.species ? a.species[j] : 0;
-          const float sig = ens_pick(a, 0, par, i, j, si, sj);
-          const float eps = ens_pick(a, 1, par, i, j, si, sj);
-          const float alp = ens_pick(a, 2, par, i, j, si, sj);
+          const float sig = ens_pick<PLAIN>(a, 0, par, i, j, si, sj);
+          const float eps = ens_pick<PLAIN>(a, 1, par, i, j, si, sj);
+          const float alp = ens_pick<PLAIN>(a, 2, par, i, j, si, sj);
           const PairD2 D = pair_eval2<JMD_SOFT_SPHERE>(r2, sig, eps, alp, a);
           if (dsig) e += 0.5 * (double)(ens_dsig(a, dsig, par, si, sj) * D.us);
           if (box) {
@@ -1058,7 +1276,7 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble_back(
     __syncthreads();
     const EnsView<STAGED> XV{tape.x, lx, a.species, lsp, S.offset};
     const EnsView<STAGED> VV{W, lv, nullptr, nullptr, S.offset};
-    double e = ens_hvp_rows(S, sp, a, par, dsig, XV, tape.idx, width, pad, VV, X, box, el);
+    double e = ens_hvp_rows<STAGED, PLAIN>(S, sp, a, par, dsig, XV, tape.idx, width, pad, VV, X, box, el);
     wg_sum3(e, el, z2, s_d);
     if (t == 0) {
       theta[sid] += e;
@@ -1067,56 +1285,103 @@ __global__ __launch_bounds__(kEnsThreads) void k_fire_ensemble_back(
     return;
   }
   double tsum = 0.0, lsum = 0.0;
+  // s1 = F'.G of the next step to be taken back: the pass that finishes P
+  // for it (3) also makes its sum, so P and F' are read once a step
+  double s1n = 0.0;
+  if (K > 0) {
+    const float keep = tape.sc[((long long)(K - 1) * nsys + sid) * kTapeScalars + 2];
+    const float* Fn = tape.F + (long long)K * n2;
+#pragma unroll 4
+    for (int m = t; m < 2 * S.n; m += nt) s1n += (double)Fn[b2 + m] * (double)keep * P[b2 + m];
+  }
   for (int k = K - 1; k >= 0; --k) {
     const float* sc = tape.sc + ((long long)k * nsys + sid) * kTapeScalars;
     const float dt = sc[0], alpha = sc[1], keep = sc[2];
     const double spp = sc[3], sff = sc[4];
     const float h = dt / 2.0f;
-    const float* Fn = tape.F + (long long)(k + 1) * n2;
-    const float* qk = tape.q + (long long)k * n2;
+    const float* __restrict__ Fn = tape.F + (long long)(k + 1) * n2;
+    const float* __restrict__ qk = tape.q + (long long)k * n2;
     // (1) FIRE mixing, backward
-    double s1 = 0.0, z1 = 0.0, z2 = 0.0;
-    for (int m = t; m < 2 * S.n; m += nt) s1 += (double)Fn[b2 + m] * (double)keep * P[b2 + m];
+    double s1 = s1n, z1 = 0.0, z2 = 0.0;
     wg_sum3(s1, z1, z2, s_d);
     const double ratio = spp / sff;
     const double cq = spp > 0.0 ? (double)alpha * s1 / (spp * sff) : 0.0;
     const double cf = (double)alpha * s1 * spp / (sff * sff * sff);
-    const float* xn = tape.x + (long long)(k + 1) * n2;
-    for (int m = t; m < 2 * S.n; m += nt) {
-      const long long g = b2 + m;
-      const double G = (double)keep * P[g];
-      const double Q = (1.0 - (double)alpha) * G + cq * (double)qk[g];
-      const double Fb = (double)alpha * ratio * G - cf * (double)Fn[g] + (double)h * Q;
-      P[g] = Q;  // PH until step (3)
-      const float vg = (float)(Fb + (double)W[g]);
-      if constexpr (STAGED) {
-        lv[m] = vg;
-        lx[m] = xn[g];
-      } else {
-        V[g] = vg;
+    const float* __restrict__ xn = tape.x + (long long)(k + 1) * n2;
+    // four elements at a time, their loads before any store (one at a time
+    // the pass waited for memory once an element)
+    for (int m0 = t; m0 < 2 * S.n; m0 += kEnsBatch * nt) {
+      double Pm[kEnsBatch];
+      float qm[kEnsBatch], Fm[kEnsBatch], Wm[kEnsBatch], xm[kEnsBatch];
+#pragma unroll
+      for (int u = 0; u < kEnsBatch; ++u) {
+        const long long g = b2 + min(m0 + u * nt, 2 * S.n - 1);
+        Pm[u] = P[g];
+        qm[u] = qk[g];
+        Fm[u] = Fn[g];
+        Wm[u] = W[g];
+        xm[u] = STAGED ? xn[g] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < kEnsBatch; ++u) {
+        const int m = m0 + u * nt;
+        if (m >= 2 * S.n) break;
+        const double G = (double)keep * Pm[u];
+        const double Q = (1.0 - (double)alpha) * G + cq * (double)qm[u];
+        const double Fb = (double)alpha * ratio * G - cf * (double)Fm[u] + (double)h * Q;
+        P[b2 + m] = Q;  // PH until step (3)
+        const float vg = (float)(Fb + (double)Wm[u]);
+        if constexpr (STAGED) {
+          lv[m] = vg;
+          lx[m] = xm[u];
+        } else {
+          V[b2 + m] = vg;
+        }
       }
     }
     __syncthreads();
     // (2) product with the force Jacobian at node k + 1
     const EnsView<STAGED> XV{xn, lx, a.species, lsp, S.offset};
     const EnsView<STAGED> VV{V, lv, nullptr, nullptr, S.offset};
-    tsum += ens_hvp_rows(S, sp, a, par, dsig, XV,
-                         tape.idx + (long long)sc[5] * ntot * width, width, pad, VV, X, box,
-                         lsum);
+    tsum += ens_hvp_rows<STAGED, PLAIN>(S, sp, a, par, dsig, XV,
+                                        tape.idx + (long long)sc[5] * ntot * width, width, pad,
+                                        VV, X, box, lsum);
     __syncthreads();
     // (3) x_{k+1} = x_k + dt ph - L m_k, ph = p_k + h F_k
-    const float* xk = tape.x + (long long)k * n2;
-    const float* xk1 = tape.x + (long long)(k + 1) * n2;
-    for (int m = t; m < 2 * S.n; m += nt) {
-      const long long g = b2 + m;
-      if (box) {
-        const float fold = rintf((xk[g] - xk1[g]) / ((m & 1) ? sp.L[1] : sp.L[0]));
-        lsum -= X[g] * (double)fold;
+    const float* __restrict__ xk = tape.x + (long long)k * n2;
+    const float* __restrict__ Fk = tape.F + (long long)k * n2;
+    const double keepn = k > 0 ? (double)sc[2 - (long long)nsys * kTapeScalars] : 0.0;
+    s1n = 0.0;
+    for (int m0 = t; m0 < 2 * S.n; m0 += kEnsBatch * nt) {
+      double Pm[kEnsBatch], Xm[kEnsBatch];
+      float Fm[kEnsBatch], xm[kEnsBatch], x1[kEnsBatch];
+#pragma unroll
+      for (int u = 0; u < kEnsBatch; ++u) {
+        const long long g = b2 + min(m0 + u * nt, 2 * S.n - 1);
+        Pm[u] = P[g];
+        Xm[u] = X[g];
+        Fm[u] = Fk[g];
+        xm[u] = x1[u] = 0.0f;
+        if (box) {
+          xm[u] = xk[g];
+          x1[u] = xn[g];
+        }
       }
-      const double PH = P[g] + (double)dt * X[g];
-      P[g] = PH;
-      W[g] = (float)((double)h * PH);
+#pragma unroll
+      for (int u = 0; u < kEnsBatch; ++u) {
+        const int m = m0 + u * nt;
+        if (m >= 2 * S.n) break;
+        if (box) {
+          const float fold = rintf((xm[u] - x1[u]) / ((m & 1) ? sp.L[1] : sp.L[0]));
+          lsum -= Xm[u] * (double)fold;
+        }
+        const double PH = Pm[u] + (double)dt * Xm[u];
+        P[b2 + m] = PH;
+        W[b2 + m] = (float)((double)h * PH);
+        s1n += (double)Fm[u] * keepn * PH;
+      }
     }
+    // end of step k, backward
     __syncthreads();
   }
   double e = tsum, el = lsum, z2 = 0.0;
@@ -1146,17 +1411,6 @@ static bool ens_lds_allow(const void* kernel, size_t* granted, size_t bytes) {
   return true;
 }
 
-static bool ens_lds_ready(size_t bytes) {
-  static size_t granted[64] = {};
-  return ens_lds_allow(reinterpret_cast<const void*>(&k_fire_ensemble<true>), granted, bytes);
-}
-
-static bool ens_lds_ready_back(size_t bytes) {
-  static size_t granted[64] = {};
-  return ens_lds_allow(reinterpret_cast<const void*>(&k_fire_ensemble_back<true>), granted,
-                       bytes);
-}
-
 int jmd_fire_ensemble_2d(const jmd_system2d* systems, const int32_t* order, int32_t n_systems,
                          int64_t n_total, int32_t mode, int32_t n_steps, double* position_hi,
                          float* position, float* momentum, float* force,
@@ -1166,8 +1420,11 @@ int jmd_fire_ensemble_2d(const jmd_system2d* systems, const int32_t* order, int3
                          uint8_t* error, int32_t* out_stat, double* energy, int32_t* builds,
                          float* tape_x, float* tape_force, float* tape_q, int32_t* tape_idx,
                          float* tape_scalars, void* stream) {
+  const int asked = mode >> 8;
+  if (mode < 0 || !ens_threads_ok(asked)) return JMD_ERR_INVALID;
+  mode &= 0xff;
   if (n_systems < 0 || n_total < 0 || n_total >= 0x7fffffff || width < 0 || n_steps < 0 ||
-      mode < ENS_FILL || mode > ENS_RUN || !fire_params)
+      mode > ENS_RUN || !fire_params)
     return JMD_ERR_INVALID;
   if (n_systems == 0) return JMD_OK;
   if (!systems || !order || !position || !scratch || !error || !builds) return JMD_ERR_INVALID;
@@ -1188,17 +1445,28 @@ int jmd_fire_ensemble_2d(const jmd_system2d* systems, const int32_t* order, int3
   // LDS copy of each system's positions, cell-sorted ids and species ids:
   // systems of up to 8 particles per thread (8 Ki per 1024-thread workgroup,
   // one per CU; 4 Ki per 512, two per CU); larger systems use global memory
-  const int threads = ens_threads(n_systems, n_total);
+  const int threads = ens_launch_threads(asked, n_systems, n_total);
   const int lds_n = threads * kEnsPerThread;
   const size_t lds_bytes = (size_t)lds_n * (2 * sizeof(float) + sizeof(uint16_t) + 1);
-  if (!ens_lds_ready(lds_bytes)) return JMD_ERR_LAUNCH;
-  hipLaunchKernelGGL(k_fire_ensemble<true>, dim3(n_systems), dim3(threads), lds_bytes,
+  // run mode with the common parameters has row loops without the general
+  // ones; the measuring and initial launches keep one form
+  const bool run = mode == ENS_RUN, plain = run && ens_plain(a);
+  const auto staged = plain ? k_fire_ensemble<true, true, true>
+                            : (run ? k_fire_ensemble<true, false, true>
+                                   : k_fire_ensemble<true, false, false>);
+  const auto memory = plain ? k_fire_ensemble<false, true, true>
+                            : (run ? k_fire_ensemble<false, false, true>
+                                   : k_fire_ensemble<false, false, false>);
+  static size_t granted[3][64] = {};
+  if (!ens_lds_allow(reinterpret_cast<const void*>(staged), granted[run + plain], lds_bytes))
+    return JMD_ERR_LAUNCH;
+  hipLaunchKernelGGL(staged, dim3(n_systems), dim3(threads), lds_bytes,
                      (hipStream_t)stream, reinterpret_cast<const EnsSys*>(systems), order,
                      n_systems, (int)n_total, mode, n_steps, position_hi, position, momentum,
                      force, reference_position, idx, width, scratch, a, prm, fire_state,
                      fire_n_pos, error, out_stat, energy, builds, tape, lds_n);
   JMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_fire_ensemble<false>, dim3(n_systems), dim3(threads), 0,
+  hipLaunchKernelGGL(memory, dim3(n_systems), dim3(threads), 0,
                      (hipStream_t)stream, reinterpret_cast<const EnsSys*>(systems), order,
                      n_systems, (int)n_total, mode, n_steps, position_hi, position, momentum,
                      force, reference_position, idx, width, scratch, a, prm, fire_state,
@@ -1209,8 +1477,12 @@ int jmd_fire_ensemble_2d(const jmd_system2d* systems, const int32_t* order, int3
 
 int jmd_fire_ensemble_max_cells(void) { return kEnsMaxCells; }
 
+int jmd_fire_ensemble_threads(int32_t n_systems, int64_t n_total, int32_t n_max) {
+  return ens_threads(n_systems, n_total, n_max);
+}
+
 int jmd_fire_ensemble_set_threads(int32_t threads) {
-  if (threads != 0 && threads != 256 && threads != 512 && threads != 1024) return JMD_ERR_INVALID;
+  if (!ens_threads_ok(threads)) return JMD_ERR_INVALID;
   g_ens_threads = threads;
   return JMD_OK;
 }
@@ -1225,8 +1497,11 @@ int jmd_fire_ensemble_adjoint_2d(const jmd_system2d* systems, int32_t n_systems,
                                  double* x_adjoint, double* p_adjoint, float* pending,
                                  float* scratch, double* theta, double* box_adjoint,
                                  float scale, void* stream) {
+  const int asked = mode >> 8;
+  if (mode < 0 || !ens_threads_ok(asked)) return JMD_ERR_INVALID;
+  mode &= 0xff;
   if (n_systems < 0 || n_total < 0 || n_total >= 0x7fffffff || width < 1 || n_steps < 0 ||
-      mode < BACK_INIT || mode > BACK_FINISH)
+      mode > BACK_FINISH)
     return JMD_ERR_INVALID;
   if (n_systems == 0) return JMD_OK;
   if (!systems || !x_adjoint || !p_adjoint || !pending || !scratch || !theta)
@@ -1242,16 +1517,21 @@ int jmd_fire_ensemble_adjoint_2d(const jmd_system2d* systems, int32_t n_systems,
                const_cast<float*>(tape_scalars), n_steps};
   // LDS copy of each system's node positions, product vector and species
   // ids (systems of up to 8 particles per thread; larger ones use memory)
-  const int threads = ens_threads(n_systems, n_total);
+  const int threads = ens_launch_threads(asked, n_systems, n_total);
   const int lds_n = threads * kEnsPerThread;
   const size_t lds_bytes = (size_t)lds_n * (4 * sizeof(float) + 1);
-  if (!ens_lds_ready_back(lds_bytes)) return JMD_ERR_LAUNCH;
-  hipLaunchKernelGGL(k_fire_ensemble_back<true>, dim3(n_systems), dim3(threads), lds_bytes,
+  const bool plain = ens_plain(a);
+  const auto staged = plain ? k_fire_ensemble_back<true, true> : k_fire_ensemble_back<true, false>;
+  const auto memory = plain ? k_fire_ensemble_back<false, true> : k_fire_ensemble_back<false, false>;
+  static size_t granted[2][64] = {};
+  if (!ens_lds_allow(reinterpret_cast<const void*>(staged), granted[plain], lds_bytes))
+    return JMD_ERR_LAUNCH;
+  hipLaunchKernelGGL(staged, dim3(n_systems), dim3(threads), lds_bytes,
                      (hipStream_t)stream, reinterpret_cast<const EnsSys*>(systems), n_systems,
                      (int)n_total, mode, n_steps, position, force, idx, width, a, dsigma, tape,
                      x_adjoint, p_adjoint, pending, scratch, theta, box_adjoint, scale, lds_n);
   JMD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_fire_ensemble_back<false>, dim3(n_systems), dim3(threads), 0,
+  hipLaunchKernelGGL(memory, dim3(n_systems), dim3(threads), 0,
                      (hipStream_t)stream, reinterpret_cast<const EnsSys*>(systems), n_systems,
                      (int)n_total, mode, n_steps, position, force, idx, width, a, dsigma, tape,
                      x_adjoint, p_adjoint, pending, scratch, theta, box_adjoint, scale, lds_n);

@@ -107,6 +107,7 @@ class SoftSphereFireEnsemble:
       r.threshold_sq = float(sp.threshold_sq)
       r.param_offset = s * block
     self._recs = recs
+    self._threads = lib.jmd_fire_ensemble_threads(S, self.n_total, max(ns, default=0)) << 8
     dev = self.device
     order = onp.argsort(-onp.asarray(ns), kind='stable').astype(onp.int32)  # largest first
     self.order = torch.as_tensor(order, device=dev)
@@ -153,8 +154,8 @@ class SoftSphereFireEnsemble:
     lib = nat.load()
     tp = tape or {}
     nat.check(lib.jmd_fire_ensemble_2d(
-        nat.ptr(self._systems), nat.ptr(self.order), len(self.sizes), self.n_total, mode,
-        n_steps, nat.ptr(self.position_hi), nat.ptr(self.position), nat.ptr(self.momentum),
+        nat.ptr(self._systems), nat.ptr(self.order), len(self.sizes), self.n_total,
+        mode | self._threads, n_steps, nat.ptr(self.position_hi), nat.ptr(self.position), nat.ptr(self.momentum),
         nat.ptr(self.force), nat.ptr(self.reference_position), nat.ptr(self.idx),
         self.width, nat.ptr(self.scratch), ctypes.byref(self._pot), self._fire,
         nat.ptr(self.fire_state), nat.ptr(self.fire_n_pos), nat.ptr(self.error),
@@ -303,7 +304,8 @@ class SoftSphereFireEnsemble:
 
     def back(mode, k):
       nat.check(lib.jmd_fire_ensemble_adjoint_2d(
-          nat.ptr(self._systems), S, self.n_total, mode, k, nat.ptr(self.position),
+          nat.ptr(self._systems), S, self.n_total, mode | self._threads, k,
+          nat.ptr(self.position),
           nat.ptr(self.force), nat.ptr(self.idx), self.width, ctypes.byref(self._pot),
           nat.ptr(dsig), nat.ptr(tape['x']), nat.ptr(tape['F']), nat.ptr(tape['q']),
           nat.ptr(tape['idx']), nat.ptr(tape['sc']), nat.ptr(X), nat.ptr(P), nat.ptr(W),

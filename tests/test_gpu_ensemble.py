@@ -285,3 +285,29 @@ def test_ensemble_large_systems_thread_counts_agree():
   print(th5, th1, lb5, lb1, flush=True)
   assert np.allclose(th5, th1, rtol=1e-6, atol=0)
   assert np.allclose(lb5, lb1, rtol=1e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize('n,L,moved', [
+    (20, 4.9, 0),      # 3 cells a side, a few ids each: three-cell runs
+    (33, 6.5, 0),      # 4 cells a side
+    (90, 4.9, 0),      # about 10 ids a cell: on either side of the mask's size
+    (300, 6.5, 0),     # cells too full for a mask: cell by cell
+    (60, 8.1, 5),      # positions outside [0, L]: the exact test throughout
+    (1100, 30.0, 0),   # more rows than threads, border runs in two pieces
+])
+def test_ensemble_rows_match_oracle(n, L, moved):
+  """The row build's forms (runs of three cells as masks; cell by cell) give
+  the oracle's list, entry for entry."""
+  jmd = _jmd()
+  rng = np.random.default_rng(n)
+  R = (rng.uniform(0, L, (n, 2))).astype(np.float32)
+  R[:moved, 0] = np.float32(L) + rng.uniform(0.01, 0.2, moved).astype(np.float32)
+  R[moved:2 * moved, 1] = -rng.uniform(0.01, 0.2, moved).astype(np.float32)
+  L = np.float32(L)
+  print('case ensemble rows', n, L, moved, flush=True)
+  ens = jmd.ensemble.SoftSphereFireEnsemble([R], [L], [np.zeros(n, np.int32)], sigma=1.4, **FIRE)
+  ens.allocate()
+  assert int(ens.did_buffer_overflow.max()) == 0
+  spec = O.NeighborListSpec(O.Space(L), L, F32(1.4), 0.2, 1.25, False, True, O.DENSE)
+  o = O.neighbor_list_build(spec, R)
+  assert np.array_equal(ens.system_neighbors(0).cpu().numpy(), o.idx)
