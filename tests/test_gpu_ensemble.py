@@ -311,3 +311,32 @@ def test_ensemble_rows_match_oracle(n, L, moved):
   spec = O.NeighborListSpec(O.Space(L), L, F32(1.4), 0.2, 1.25, False, True, O.DENSE)
   o = O.neighbor_list_build(spec, R)
   assert np.array_equal(ens.system_neighbors(0).cpu().numpy(), o.idx)
+
+
+@pytest.mark.parametrize('sizes,threads', [([128, 300], 512), ([97, 900], 1024)])
+def test_ensemble_general_form_matches_plain_fire(sizes, threads):
+  """alpha other than 2 takes the run instance with the general pair forms,
+  at either side of the rule for threads per system; bars as for alpha = 2."""
+  jmd = _jmd()
+  from jax_md_amd import _native as nat
+  assert nat.load().jmd_fire_ensemble_threads(len(sizes), sum(sizes), max(sizes)) == threads
+  syst = _systems(sizes, seed=23)
+  print('case ensemble general', sizes, flush=True)
+  ens = jmd.ensemble.SoftSphereFireEnsemble([s[0] for s in syst], [s[2] for s in syst],
+                                            [s[1] for s in syst], sigma=SIGMA, alpha=2.5, **FIRE)
+  ens.allocate().run(20)
+  assert int(ens.did_buffer_overflow.max()) == 0
+  for s, (R, sp, L) in enumerate(syst):
+    disp, shift = jmd.space.periodic(L)
+    nfn, efn = jmd.energy.soft_sphere_neighbor_list(
+        disp, L, species=torch.as_tensor(sp, device=DEV), alpha=2.5,
+        sigma=torch.as_tensor(SIGMA, device=DEV), format=jmd.partition.Dense)
+    init_fn, apply_fn = jmd.minimize.fire_descent(efn, shift, **FIRE)
+    Rt = torch.as_tensor(R, device=DEV)
+    nb = nfn.allocate(Rt)
+    st = init_fn(Rt, neighbor=nb)
+    for _ in range(20):
+      nb = nb.update(st.position)
+      st = apply_fn(st, neighbor=nb)
+    dx = (ens.position_hi[ens.system_slice(s)] - st.position_hi).abs().max().item()
+    assert dx <= 1e-5, (s, dx)
