@@ -54,7 +54,7 @@ __device__ __forceinline__ float fast_rsqrt(float x) {
 // t = (sigma^2/r^2)^3, A = t - 1, B = 2 t - 1 and, for the switch,
 //   y = clamp((rc^2 - r^2) / (rc^2 - ro^2), 0, 1),  x = 1 - y,
 //   S = y^2 (3 - 2 y),  S'/r = -12 x y / (rc^2 - ro^2):
-//   v = S t A,  g = t y [ y (3 - 2 y) B / r^2 + 2 x A / (rc^2 - ro^2) ].
+//   v = S (t^2 - t),  g = t y [ y (3 - 2 y) B / r^2 + 2 x A / (rc^2 - ro^2) ].
 // The clamp covers all three regions (y = 1: plain, y = 0: beyond the
 // cutoff) and costs nothing on the product; the common factor t y is
 // taken out, so a pair is 18 operations from r^2 to g.  The caller applies
@@ -74,6 +74,7 @@ __device__ __forceinline__ float lj_reduced(float r2, float sig2, const PairArgs
   const float s2 = sig2 * inv_r2;
   const float t = s2 * s2 * s2;
   const float B = fmaf(2.0f, t, -1.0f);
+  const float w = fmaf(t, t, -t);  // not t (t - 1): no number at r = 0, where t is infinite
   if (SMOOTH == 1 || (SMOOTH < 0 && a.smooth)) {
     const float y = __builtin_amdgcn_fmed3f((a.rc2 - r2) * a.sw, 0.0f, 1.0f);
     const float x = 1.0f - y;
@@ -81,11 +82,11 @@ __device__ __forceinline__ float lj_reduced(float r2, float sig2, const PairArgs
     const float A2 = fmaf(t, a.sw2, -a.sw2);  // 2 A / (rc^2 - ro^2)
     const float q = fmaf(z, B * inv_r2, x * A2);
     const float ty = t * y;
-    *v = z * ty * (t - 1.0f);
+    *v = z * y * w;
     return q * ty;
   }
   const bool valid = r2 < a.rc2;
-  *v = valid ? t * (t - 1.0f) : 0.0f;
+  *v = valid ? w : 0.0f;
   return valid ? t * (B * inv_r2) : 0.0f;
 }
 
