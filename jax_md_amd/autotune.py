@@ -8,7 +8,7 @@ the largest row (partition.py:1092-1104, ``capacity_multiplier``); XLA picks
 its own fusion layout for the pair reduction.  Here:
 
 - ``threads_per_atom`` (lanes per Dense row in the force pass) is a knob of
-  the pair kernel (``jmd_set_threads_per_atom``);
+  the pair kernel (``jmd_set_threads_per_atom``), 0 its built-in rule by size;
 - ``cell_size_factor`` makes cells at least that multiple of the list cutoff
   (``partition.neighbor_list(..., cell_size_factor=)``): the neighbour sets
   are the same, the rows follow that grid's candidate order;
@@ -20,7 +20,9 @@ copies of the given state, by coordinate descent: threads per row first, then
 the cell size, then the capacity.  A candidate whose list overflows during
 its trial is discarded.  Results are cached per workload (particle count,
 dimension, density, cutoffs, list format, potential) for the process, and in
-a JSON file when ``cache_path`` is given.
+a JSON file when ``cache_path`` is given; an entry of the file is taken as it
+was saved (one made before the kernel's rule was among the candidates keeps
+its setting until it is deleted).
 """
 
 from __future__ import annotations
@@ -42,7 +44,8 @@ _current_tpa = 0  # threads per row the library was last told (0: its built-in c
 
 def set_threads_per_atom(tpa: int) -> None:
   """Lanes per Dense row of the force pass for every later launch in this
-  process (0 restores the built-in choice: 8 in 3-D, 2 in 2-D)."""
+  process: 2, 4, 8 or 16; 0 restores the built-in choice, in 3-D 32, 16 or 8
+  by the number of rows and their width, in 2-D 2."""
   global _current_tpa
   nat.check(nat.load().jmd_set_threads_per_atom(int(tpa)), 'jmd_set_threads_per_atom')
   _current_tpa = int(tpa)
@@ -50,7 +53,7 @@ def set_threads_per_atom(tpa: int) -> None:
 
 @dataclasses.dataclass
 class TunedConfig:
-  threads_per_atom: int
+  threads_per_atom: int  # 0: the kernel's built-in rule
   cell_size_factor: float
   capacity_multiplier: float
   us_per_step: float
@@ -134,7 +137,7 @@ def _time_trial(make_fns, position, momentum, shift_fn, dt, kwargs, tpa, trial_s
 
 def tune_nve_loop(make_fns: Callable, position: torch.Tensor, momentum: torch.Tensor,
                   shift_fn, dt: float, key: Optional[tuple] = None, trial_steps: int = 40,
-                  repeats: int = 3, tpas: Sequence[int] = (4, 8, 16),
+                  repeats: int = 3, tpas: Sequence[int] = (0, 4, 8, 16),
                   cell_size_factors: Sequence[float] = (1.0, 1.15, 1.3),
                   capacity_multipliers: Sequence[float] = (1.25, 1.5),
                   cache_path: Optional[str] = None) -> TunedConfig:
@@ -145,6 +148,9 @@ def tune_nve_loop(make_fns: Callable, position: torch.Tensor, momentum: torch.Te
   list and potential with the given ``cell_size_factor`` and
   ``capacity_multiplier`` (e.g. ``lambda **kw:
   energy.lennard_jones_neighbor_list(disp, box, format=Dense, **kw)``).
+  ``tpas`` holds 0, the kernel's own rule, so that a tuned loop is not slower
+  than an untuned one (the rule's 32 lanes for small systems have no setting
+  of their own).
   ``position`` / ``momentum`` are the state to time from; they are not
   modified.  ``key`` (see ``workload_key``) caches the result; the process
   keeps its threads-per-row setting as it was.
@@ -161,8 +167,8 @@ def tune_nve_loop(make_fns: Callable, position: torch.Tensor, momentum: torch.Te
     _CACHE[key] = cfg
     return cfg
   saved_tpa = _current_tpa
-  default_tpa = 8 if position.shape[1] == 3 else 2
-  best = {'tpa': default_tpa if default_tpa in tpas else tpas[0],
+  starts = (0, 8 if position.shape[1] == 3 else 2)
+  best = {'tpa': next((t for t in starts if t in tpas), tpas[0]),
           'cell_size_factor': cell_size_factors[0],
           'capacity_multiplier': (1.25 if 1.25 in capacity_multipliers
                                   else capacity_multipliers[0])}

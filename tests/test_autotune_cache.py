@@ -1,5 +1,5 @@
 """The autotuner's host side, without a GPU: its cache key (density from
-scalar, vector and matrix boxes) and its JSON file cache."""
+scalar, vector and matrix boxes), its JSON file cache and its candidates."""
 
 import numpy as np
 
@@ -26,3 +26,26 @@ def test_autotune_workload_key_and_file_cache(tmp_path):
   assert (cfg.threads_per_atom, cfg.cell_size_factor, cfg.capacity_multiplier) == (16, 1.15, 1.5)
   assert cfg.neighbor_kwargs == {'cell_size_factor': 1.15, 'capacity_multiplier': 1.5}
   autotune._CACHE.clear()
+
+
+def test_tuner_keeps_the_built_in_lanes_where_they_are_the_fastest(monkeypatch):
+  """The kernel's own rule (0; 32 lanes for small systems, which no setting
+  names) is among the candidates and is what the tuner starts from."""
+  import torch
+  from jax_md_amd import autotune
+  us = {0: 13.9, 4: 18.0, 8: 16.5, 16: 14.7}  # N = 4,096: the rule beats every setting
+  set_to = []
+  monkeypatch.setattr(autotune, 'set_threads_per_atom', set_to.append)
+  monkeypatch.setattr(
+      autotune, '_time_trial',
+      lambda make, R, P, shift, dt, kw, tpa, steps, reps:
+      us[tpa] * kw['cell_size_factor'] * kw['capacity_multiplier'])
+  R = torch.zeros((4096, 3))
+  cfg = autotune.tune_nve_loop(None, R, R, None, 0.005)
+  assert (cfg.threads_per_atom, cfg.cell_size_factor, cfg.capacity_multiplier) == (0, 1.0, 1.25)
+  cfg.apply()
+  assert set_to[-1] == 0
+  # every candidate overflows: the settings the library has without tuning
+  monkeypatch.setattr(autotune, '_time_trial', lambda *a: None)
+  cfg = autotune.tune_nve_loop(None, R, R, None, 0.005)
+  assert (cfg.threads_per_atom, cfg.cell_size_factor, cfg.capacity_multiplier) == (0, 1.0, 1.25)
