@@ -264,19 +264,25 @@ __global__ __launch_bounds__(256) void k_pair_dense(
   row_sum<DIM, STRIDE, KIND, TPA, GENERAL, ENERGY, SM, BX, F32, U>(pos, n, s, a, row, \
                                                                    width, sub, i, xi, near, \
                                                                    f, &e)
-#define JMD_ROW_SM(BX, F32)                                                      \
+#define JMD_ROW_SM(BX, F32, U)                                                   \
   do {                                                                           \
-    if (KIND == JMD_LENNARD_JONES && a.smooth) JMD_ROW(1, BX, F32, 4);           \
-    else JMD_ROW(0, BX, F32, 4);                                                 \
+    if (KIND == JMD_LENNARD_JONES && a.smooth) JMD_ROW(1, BX, F32, U);           \
+    else JMD_ROW(0, BX, F32, U);                                                 \
   } while (0)
+    // Tables beyond 2 GiB (134 million 16-byte rows) are gathered by address.
+    // Four entries in flight as below, two where the registers of four
+    // addresses would cost every launch of the instance a wavefront per SIMD.
+    // 134,479,872 rows of 26 entries (scalar and species Lennard-Jones, soft
+    // sphere): 8.9, 16.4 and 9.5 ms; 10.6, 18.3 and 11.6 with one in flight and
+    // the switch tested per pair.
+    constexpr int kWideUnr = !GENERAL && (KIND == JMD_LENNARD_JONES || DIM == 3) ? 4 : 2;
     if ((long long)n * (STRIDE * 4) > 0x7fffffffLL) {
-      // (more than 134 million rows: the compact form)
-      if (s.general) JMD_ROW(-1, true, false, 1);
-      else JMD_ROW(-1, false, false, 1);
+      if (s.general) JMD_ROW_SM(true, false, kWideUnr);
+      else JMD_ROW_SM(false, false, kWideUnr);
     } else if (s.general) {
-      JMD_ROW_SM(true, true);
+      JMD_ROW_SM(true, true, 4);
     } else {
-      JMD_ROW_SM(false, true);
+      JMD_ROW_SM(false, true, 4);
     }
 #undef JMD_ROW_SM
 #undef JMD_ROW
