@@ -241,3 +241,36 @@ def test_chain_half_steps_vs_oracle(rate, substeps, mode):
           abs(float(kin) - ke2) / ke2, abs(float(scale) - s) / s)
   print(f'  rel errors p_xi {errs[0]:.2e} xi {errs[1]:.2e} ke {errs[2]:.2e} scale {errs[3]:.2e}')
   assert all(np.isfinite(errs)) and max(errs) < tol
+
+
+@pytest.mark.parametrize('nparts', [1, 255, 257, 1792, 1793, 2049, 4096, 8195])
+def test_kinetic_partials_are_summed_in_their_order(nparts):
+  """The kinetic energy of jmd_nhc_step from its partials, bit for bit in the
+  stated order (thread t adds t, t + 256, ..., then a tree), on both sides of
+  the counts where a thread has eight loads in flight (more than 458,752
+  particles)."""
+  print(f'case kinetic partials {nparts}', flush=True)
+  jmd = _jmd()
+  nat = jmd._native
+  lib = nat.load()
+  part = np.random.default_rng(nparts).normal(size=nparts) * 10.0 ** (np.arange(nparts) % 7)
+  lanes = np.zeros(256)
+  for b in range(0, nparts, 256):
+    lanes[:min(256, nparts - b)] += part[b:b + 256]
+  off = 128
+  while off:
+    lanes[:off] += lanes[off:2 * off]
+    off //= 2
+  L, n = 5, 100
+  chain = torch.zeros((3, L), dtype=torch.float64, device=DEV)
+  kin, scale = (torch.zeros((1,), dtype=torch.float64, device=DEV) for _ in range(2))
+  part_d = torch.as_tensor(part, device=DEV)
+  nat.check(lib.jmd_nhc_step(4, nat.ptr(chain), L, 2, 3, 0.005, 1.0, 0.5, 3.0 * n, nat.ptr(kin),
+                             nat.ptr(part_d), nparts, nat.ptr(scale),
+                             nat.stream_handle(chain.device)), 'jmd_nhc_step')
+  assert float(kin) == lanes[0]
+
+
+def test_fused_kick_with_many_workgroups_equals_two_launches():
+  """As above for n = 600,001 (2,344 partials)."""
+  test_fused_kick_kinetic_chain_equals_two_launches(600001, 3)
