@@ -231,13 +231,22 @@ static int g_tpa_override = 0;
 // rows are long enough to feed them.  A 20-step block of Lennard-Jones rows
 // of 95 entries, us with 8 / 16 / 32 lanes: 330 / 293 / 278 (N = 4,096),
 // 330 / 299 / 296 (8,000), 375 / 361 / 384 (15,625), 417 / 408 / 441 (22,736),
-// 463 / 478 / 519 (32,768).  2-D rows (a few entries) get 2.
-static int lanes_per_row(int dim, int64_t n, int64_t width) {
+// 463 / 478 / 519 (32,768).  The 16 lanes end earlier, us with 8 / 16:
+// - for narrow rows (34 to 38 entries; scalar and species Lennard-Jones,
+//   scalar and species soft spheres): 218 / 216, 224 / 219, 211 / 209 and
+//   222 / 211 at 12,167 rows, 222 / 225, 228 / 232, 214 / 218 and 224 / 229 at
+//   15,625, 228 / 237, 240 / 246, 223 / 228 and 234 / 276 at 21,952;
+// - for other than scalar parameters: the soft-sphere instance then holds 5
+//   wavefronts a SIMD, 5,120 on the chip, which 16 lanes of 20,480 rows
+//   are (species soft spheres of 67 entries 294 / 270 at 19,683 rows and
+//   294 / 331 at 21,952, scalar ones there 267 / 264).
+// 2-D rows (a few entries) get 2.
+static int lanes_per_row(int dim, int64_t n, int64_t width, bool general) {
   if (g_tpa_override) return g_tpa_override;
   if (dim == 2) return 2;
   if (n <= 8192 && width >= 64) return 32;
-  if (n <= 24576 && width >= 32) return 16;
-  return 8;
+  const int64_t most = width >= 64 ? (general ? 20480 : 24576) : 12288;
+  return n <= most && width >= 32 ? 16 : 8;
 }
 
 constexpr long long kSparseBlocks = 2048;
@@ -461,7 +470,7 @@ int pair_energy_force(const float* position, int64_t n, int32_t dim, int32_t pos
       }
       return JMD_OK;
     }
-    const int tpa = lanes_per_row(dim, n, idx_width);
+    const int tpa = lanes_per_row(dim, n, idx_width, a.general);
     long long threads = (long long)nn * tpa;
     int nb = ceil_div(threads, 256);
     nb = (nb + 7) & ~7;
@@ -651,7 +660,7 @@ int jmd_nve_force_kick_drift(const float* position, int64_t n, int32_t dim,
   box_inverse(kd.s, kd.Ti);
   hipStream_t st = (hipStream_t)stream;
   const int nn = (int)n;
-  const int tpa = lanes_per_row(dim, n, idx_width);
+  const int tpa = lanes_per_row(dim, n, idx_width, a.general);
   int nb = ceil_div((long long)nn * tpa, 256);
   nb = (nb + 7) & ~7;
   DenseLaunch L{dim3(nb), st, position, nn, s, a, idx, (int)idx_width, force, nullptr,

@@ -16,16 +16,22 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 
 
-def _rows_fp64(R, sides, idx):
-  """Energy and force of the switched Lennard-Jones rows in float64."""
+def _rows_fp64(R, sides, idx, species=None, sigma=1.0):
+  """Energy and force of the switched Lennard-Jones rows in float64; sides is
+  a vector, or a box matrix with R fractional."""
   x, L = R.astype(np.float64), np.asarray(sides, np.float64)
   n = len(x)
   i, k = np.nonzero(idx < n)
-  d = x[idx[i, k]] - x[i]
-  d -= L * np.rint(d / L)
+  j = idx[i, k]
+  d = x[j] - x[i]
+  if L.ndim == 2:
+    d = (d - np.rint(d)) @ L.T
+  else:
+    d -= L * np.rint(d / L)
   s = (d ** 2).sum(1)
   c, o = 2.5 ** 2, 2.0 ** 2
-  q6 = s ** -3.0
+  sig = sigma if species is None else np.asarray(sigma, np.float64)[species[i], species[j]]
+  q6 = (sig ** 2 / s) ** 3.0
   V, dV = 4 * (q6 ** 2 - q6), -24 * (2 * q6 ** 2 - q6) / s
   S = np.where(s < o, 1.0, (c - s) ** 2 * (c + 2 * s - 3 * o) / (c - o) ** 3)
   dS = np.where(s < o, 0.0, 12 * (c - s) * (o - s) / (c - o) ** 3)
@@ -96,3 +102,36 @@ def test_energy_total_is_the_sum_of_its_rows(n):
   E, _ = efn.energy_and_force(R, nbrs)
   each = each_fn(R, nbrs).to(torch.float64)
   assert abs(float(E) - float(each.sum())) <= 2.0 ** -24 * float(each.abs().sum()) + 1e-30
+
+
+@pytest.mark.parametrize('n', [8192, 8193, 12288, 12289, 20480, 20481, 24576, 24577])
+@pytest.mark.parametrize('spacing,skin,species', [(1.06, 0.5, False), (1.06, 0.5, True),
+                                                  (1.36, 0.3, False)])
+def test_rows_on_both_sides_of_the_lane_rule(n, spacing, skin, species):
+  """The built-in lanes at the row counts where they change: wide rows of
+  scalar and of species parameters, narrow rows."""
+  import jax_md_amd as jmd
+  rng = np.random.default_rng(n)
+  dims = (30, 29, 29)
+  sides = (np.array(dims) * spacing).astype(np.float32)
+  g = np.stack(np.meshgrid(*[np.arange(d) for d in dims], indexing='ij'), -1).reshape(-1, 3)
+  R = ((g[:n] + 0.5) * spacing + rng.uniform(-0.08, 0.08, (n, 3))).astype(np.float32)
+  sp, sig = None, np.float32(1.0)
+  kw = {}
+  if species:
+    sp = rng.integers(0, 2, n).astype(np.int32)
+    sig = np.array([[1.0, 0.95], [0.95, 0.9]], np.float32)
+    kw = dict(species=torch.as_tensor(sp, device=DEV), sigma=torch.as_tensor(sig, device=DEV))
+  disp, _ = jmd.space.periodic(sides)
+  nfn, efn = jmd.energy.lennard_jones_neighbor_list(disp, sides, format=jmd.partition.Dense,
+                                                    dr_threshold=skin, **kw)
+  Rt = torch.as_tensor(R, device=DEV)
+  nbrs = nfn.allocate(Rt)
+  assert nbrs.idx.shape[1] >= 64 if spacing < 1.2 else 32 <= nbrs.idx.shape[1] < 64
+  E64, F64 = _rows_fp64(R, sides, nbrs.idx.cpu().numpy(), sp, sig)
+  E, F = efn.energy_and_force(Rt, nbrs)
+  rel, worst = _force_err(F.cpu().numpy(), F64)
+  print(f'lane rule n={n} width {nbrs.idx.shape[1]} species {species}: {rel:.2e} {worst:.2e}',
+        flush=True)
+  assert rel <= FORCE_RTOL and worst <= FORCE_WORST
+  assert abs(float(E) - E64) <= 1e-6 * abs(E64)
