@@ -252,6 +252,9 @@ int jmd_set_threads_per_atom(int32_t threads_per_atom);
  *                                    Dense and Sparse only)
  *   energy_total   [1]      float64  total energy, summed in float64
  * Pair arithmetic is float32 with float64 per-particle accumulation.
+ * Dense rows hold their entries first and n (or more) after them, as
+ * jmd_neighbor_list_build leaves them: whether an entry after a gap counts is
+ * not defined (here, in the VJP, the virial and the float64 form).
  * When momentum is non-NULL (force required) the call also applies
  * p += half_dt * F (the closing half kick of simulate.velocity_verlet,
  * simulate.py:240-241): in the same pass for Dense lists, in a second

@@ -386,7 +386,10 @@ def pair_neighbor_list(fn, displacement_or_metric, species=None,
                        reduce_axis: Optional[Tuple[int, ...]] = None,
                        ignore_unused_parameters: bool = False, **kwargs) -> PairEnergy:
   """Promotes a pair function to a neighbour-list energy
-  (jax_md/smap.py:856-979)."""
+  (jax_md/smap.py:856-979).  Dense rows are read as ``partition`` leaves them,
+  entries first and padding N after them; to drop pairs from a row, use
+  ``custom_mask_function`` (or close the gaps): whether an entry after a gap
+  counts is not defined."""
   kind, r_on, r_c = _native_kind(fn)
   kwargs = dict(kwargs)
   # the reference passes it on to the pair function, which ignores it

@@ -1,7 +1,7 @@
 """The Dense row kernel at the edges of its blocks: every lane count, row
-widths that end inside and at a block, rows of wavefronts on and off the box
-faces, padding entries in the middle of a row, boxes whose faces are near in
-some dimensions only.  Forces against the float64 sum over the same rows, with
+widths that end inside and at a block, rows that end anywhere beside longer
+ones, rows of wavefronts on and off the box faces, boxes whose faces are near in
+some dimensions only, species parameters and box matrices.  Forces against the float64 sum over the same rows, with
 the bars of test_gpu_pair.py (float32 pair terms: 1e-5 norm-wise, 5e-5 of the
 rms for one particle, 1e-6 for the energy)."""
 
@@ -9,7 +9,6 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import jaxmd_oracle as O
 from tests.test_gpu_pair import FORCE_RTOL, FORCE_WORST, _force_err
 
 pytestmark = pytest.mark.gpu
@@ -53,12 +52,12 @@ def _system(dims, seed):
 
 
 @pytest.mark.parametrize('lanes', [0, 2, 4, 8, 16])
-@pytest.mark.parametrize('dims,multiplier,holes', [
+@pytest.mark.parametrize('dims,multiplier,shortened', [
     ((8, 8, 8), 1.0, False),       # all pairs, rows end at their capacity
     ((9, 8, 14), 1.25, True),      # far faces in one dimension only
     ((11, 13, 10), 1.0, False),
     ((16, 9, 9), 1.5, True)])
-def test_rows(lanes, dims, multiplier, holes):
+def test_rows(lanes, dims, multiplier, shortened):
   import jax_md_amd as jmd
   R, sides = _system(dims, seed=sum(dims))
   disp, _ = jmd.space.periodic(sides)
@@ -66,10 +65,10 @@ def test_rows(lanes, dims, multiplier, holes):
                                                     capacity_multiplier=multiplier)
   Rt = torch.as_tensor(R, device=DEV)
   nbrs = nfn.allocate(Rt)
-  if holes:  # a caller that drops pairs by writing N over them
-    rng = np.random.default_rng(1)
-    drop = torch.as_tensor(rng.random(tuple(nbrs.idx.shape)) < 0.1, device=DEV)
-    nbrs.idx[drop] = R.shape[0]
+  if shortened:  # rows of any length in one wavefront, empty ones among them
+    keep = np.random.default_rng(1).integers(0, nbrs.idx.shape[1] + 1, (R.shape[0], 1))
+    past = torch.arange(nbrs.idx.shape[1], device=DEV) >= torch.as_tensor(keep, device=DEV)
+    nbrs.idx[past] = R.shape[0]
   E64, F64 = _rows_fp64(R, sides, nbrs.idx.cpu().numpy())
   lib = jmd._native.load()
   assert lib.jmd_set_threads_per_atom(lanes) == 0
@@ -85,10 +84,51 @@ def test_rows(lanes, dims, multiplier, holes):
     lib.jmd_set_threads_per_atom(0)
 
 
-@pytest.mark.parametrize('n', [1, 63, 4096, 32184, 70001])
+@pytest.mark.parametrize('lanes', [0, 2, 4, 8, 16])
+@pytest.mark.parametrize('species,matrix', [(True, False), (False, True), (True, True)])
+def test_rows_with_species_and_box_matrix(lanes, species, matrix):
+  """Parameters by species and fractional positions in a triclinic box, whose
+  rows take their own instances and folds."""
+  import jax_md_amd as jmd
+  R, sides = _system((11, 9, 10), seed=3)
+  n = R.shape[0]
+  rng = np.random.default_rng(4)
+  kw, sp, sig = {}, None, np.float32(1.0)
+  if species:
+    sp = rng.integers(0, 2, n).astype(np.int32)
+    sig = np.array([[1.0, 0.95], [0.95, 0.9]], np.float32)
+    kw = dict(species=torch.as_tensor(sp, device=DEV), sigma=torch.as_tensor(sig, device=DEV))
+  box, disp = sides, jmd.space.periodic(sides)[0]
+  if matrix:
+    box = np.diag(sides) + np.array([[0, 1.1, 0.4], [0, 0, 0.9], [0, 0, 0]], np.float32)
+    R = (R / sides).astype(np.float32)
+    disp = jmd.space.periodic_general(box)[0]
+    kw['fractional_coordinates'] = True
+  nfn, efn = jmd.energy.lennard_jones_neighbor_list(disp, box, format=jmd.partition.Dense, **kw)
+  Rt = torch.as_tensor(R, device=DEV)
+  nbrs = nfn.allocate(Rt)
+  E64, F64 = _rows_fp64(R, box, nbrs.idx.cpu().numpy(), sp, sig)
+  lib = jmd._native.load()
+  assert lib.jmd_set_threads_per_atom(lanes) == 0
+  try:
+    for in_box in (False, True):
+      F = efn.force(Rt, nbrs, in_box=in_box)
+      rel, worst = _force_err(F.cpu().numpy(), F64)
+      print(f'rows species {species} matrix {matrix} lanes {lanes} in_box {in_box}: '
+            f'{rel:.2e} {worst:.2e}', flush=True)
+      assert rel <= FORCE_RTOL and worst <= FORCE_WORST
+    E, _ = efn.energy_and_force(Rt, nbrs)
+    assert abs(float(E) - E64) <= 1e-6 * abs(E64)
+  finally:
+    lib.jmd_set_threads_per_atom(0)
+
+
+@pytest.mark.parametrize('n', [1, 63, 4096, 32184, 70001, 98304, 98305, 131073, 262177, 600000])
 def test_energy_total_is_the_sum_of_its_rows(n):
   """The total over block partials against the particles' own energies
-  (float32 each, summed here in float64): 2^-24 of the sum of magnitudes."""
+  (float32 each, summed here in float64): 2^-24 of the sum of magnitudes.
+  The last five have 3,072 partials, up to which a thread of the sum takes them
+  one at a time, and 3,080, 4,104, 8,200 and 18,752, which it takes by fours."""
   import jax_md_amd as jmd
   g = torch.Generator(device=DEV).manual_seed(n)
   R = torch.rand((n, 3), generator=g, device=DEV) * 100.0
