@@ -33,7 +33,7 @@ namespace jmd {
 constexpr int kEnsThreads = 1024;  // the most a workgroup has
 constexpr int kEnsWaves = 4;       // a SIMD (at 8, 64 VGPRs: the run spilled and took 1.5 times as long)
 static int g_ens_threads = 0;      // jmd_fire_ensemble_set_threads (0: by size)
-constexpr int kEnsCUs = 256;
+constexpr int kEnsCUs = 256;       // of an MI355X
 inline int ens_threads(int n_systems, long long n_total, long long n_max) {
   if (n_systems > 0 && n_total / n_systems >= 4096) return 1024;
   return n_max >= 768 && n_max >= n_total / kEnsCUs ? 1024 : 512;
@@ -512,10 +512,11 @@ __device__ __forceinline__ int ens_rows(const EnsSys& S, const Grid& g, const Sp
                         const uint16_t* ls, bool all_in, int fill) {
   const int nt = blockDim.x, t = threadIdx.x;
   // The candidate test: the minimum-image |x_j - x_i|^2 of positions in the
-  // box decides every candidate farther than `margin` from the cutoff (the
-  // bound of the main cell build on the few float32 roundings by which it
-  // can differ from the reference's wrapped float32 d^2); the rest, and
-  // positions outside [0, L], take the reference-exact two-way test.
+  // box decides every candidate farther than `margin` from the cutoff; the
+  // rest, and positions outside [0, L], take the reference-exact two-way test.
+  // The few float32 roundings by which it can differ from the reference's
+  // wrapped float32 d^2 are bounded where the cell build sets its margin;
+  // this one is four times that bound.
   const float rc = sqrtf(cutoff_sq), Lmax = fmaxf(sp.L[0], sp.L[1]);
   const float margin =
       fmaxf(128.0f * (rc + 1.0f) * (Lmax + rc + 1.0f) * 1.1920929e-7f, 1e-4f * cutoff_sq);

@@ -135,7 +135,7 @@ __device__ const double kSYWeights[4][7] = {
 constexpr int kMaxChain = 16;
 
 // exp(x) in float64: the chain's arguments are small (|x| << 0.05), where
-// nine Taylor terms are exact to rounding (x^10/10! < 1e-22 relative at 1/32)
+// nine Taylor terms are exact to rounding (x^10/10! < 3e-22 relative at 1/32)
 // and several times cheaper than the library call on one thread.  Horner with
 // the factorials as coefficients: one multiply-add a term.  The library call
 // stays out of line: the chain runs once a step on one lane with a cold
