@@ -52,7 +52,7 @@ __device__ __forceinline__ rsrc_t row_table(const float* p, unsigned rows, int r
 // Step kernel at N = 262,144: 48.4 -> 45 us; energy and force of 1,029,897
 // particles not known to lie in the box: 202 -> 176 us.
 template <int DIM, int STRIDE, int KIND, int TPA, bool GENERAL, bool ENERGY, int SMOOTH,
-          bool BOX, bool INDEXED, int UNR>
+          int BOX, bool INDEXED, int UNR>
 __device__ __forceinline__ void row_sum(const float* __restrict__ pos, unsigned n,
                                         const Space& s, const PairArgs& a,
                                         const int* __restrict__ row, int width, int sub,
@@ -127,7 +127,7 @@ __device__ __forceinline__ void row_sum(const float* __restrict__ pos, unsigned 
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-      if (BOX) box_apply<DIM>(s, d[u]);
+      if (BOX == 1 || (BOX < 0 && s.general)) box_apply<DIM>(s, d[u]);
       term(jj[u], d[u], square(d[u]), false, true);
     }
   };
@@ -140,7 +140,7 @@ __device__ __forceinline__ void row_sum(const float* __restrict__ pos, unsigned 
       d[c] = (near >> c) & 1u
                  ? min_image_any(xj[c], xi[c], xi[c] - s.L[c], s.L[c], s.half[c], s.inbox)
                  : xj[c] - xi[c];
-    if (BOX) box_apply<DIM>(s, d);
+    if (BOX == 1 || (BOX < 0 && s.general)) box_apply<DIM>(s, d);
     term(ok ? jraw : i, d, square(d), true, ok);
   };
   // This lane's entries are sub, sub + TPA, ... < width, in blocks of UNR
@@ -164,8 +164,32 @@ __device__ __forceinline__ void row_sum(const float* __restrict__ pos, unsigned 
         v[u] = (unsigned)row[min((int)(b * (UNR * TPA)) + u * TPA + sub, width - 1)];
     }
   };
+  if (nfull == 0) {
+    // Rows of less than a block: no loads but those of the entries there are.
+    // (Taken as a short block, soft spheres in 2-D, rows of 5 on 2 lanes, loaded
+    // twice what they needed: a force of 1,000,000 rows 17.5 us, now 12.9; in
+    // 3-D, rows of 11 on 8 lanes, 512,000 of them 24.4 and 21.5.)
+    unsigned jj[UNR];
+    float xj[UNR][3];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      jj[u] = n;
+      if (u * TPA < width) jj[u] = (unsigned)row[min(u * TPA + sub, width - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      if (u * TPA + sub >= width) jj[u] = n;
+      xj[u][0] = xj[u][1] = xj[u][2] = 0.0f;
+      if (u * TPA < width) gather(jj[u], xj[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      if (__builtin_amdgcn_ballot_w64(jj[u] < n) != 0ull) masked_entry(jj[u], xj[u]);
+    }
+    return;
+  }
   unsigned nxt[UNR];
-  if (nblk > 0) entries(0, nxt);
+  entries(0, nxt);
   for (unsigned b = 0; b < nblk; ++b) {
     unsigned jj[UNR], jmin = n, jmax = 0u;
 #pragma unroll
@@ -277,12 +301,11 @@ __global__ __launch_bounds__(256) void k_pair_dense(
     // the switch tested per pair.
     constexpr int kWideUnr = !GENERAL && (KIND == JMD_LENNARD_JONES || DIM == 3) ? 4 : 2;
     if ((long long)n * (STRIDE * 4) > 0x7fffffffLL) {
-      if (s.general) JMD_ROW_SM(true, false, kWideUnr);
-      else JMD_ROW_SM(false, false, kWideUnr);
+      JMD_ROW_SM(-1, false, kWideUnr);
     } else if (s.general) {
-      JMD_ROW_SM(true, true, 4);
+      JMD_ROW_SM(1, true, 4);
     } else {
-      JMD_ROW_SM(false, true, 4);
+      JMD_ROW_SM(0, true, 4);
     }
 #undef JMD_ROW_SM
 #undef JMD_ROW

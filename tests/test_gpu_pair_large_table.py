@@ -49,7 +49,7 @@ def _pair_fp64(kind, s, sig):
   return torch.where(s < c, S * V, 0 * s), torch.where(s < c, S * dV + dS * V, 0 * s)
 
 
-@pytest.mark.parametrize('kind', ['lj', 'lj species', 'soft'])
+@pytest.mark.parametrize('kind', ['lj', 'lj species', 'lj matrix', 'soft'])
 def test_rows_of_a_large_table(kind):
   import jax_md_amd as jmd
   if torch.cuda.get_device_properties(0).total_memory < 64 << 30:
@@ -60,11 +60,19 @@ def test_rows_of_a_large_table(kind):
   print(f'case large table {kind} n={n}', flush=True)
   box = [SPACING * d + 20.0 for d in SIDE]
   disp, _ = jmd.space.periodic(box)
-  sig = torch.tensor([[1.0, 0.95], [0.95, 0.9]], device=DEV)
+  T = torch.diag(torch.tensor(box, dtype=torch.float64, device=DEV))
   kw = dict(format=jmd.partition.Dense)
+  if kind == 'lj matrix':  # fractional positions, the lattice sheared a little
+    R /= torch.tensor(box, device=DEV)
+    T[0, 1], T[1, 2] = 0.02 * T[1, 1], 0.03 * T[2, 2]
+    T = T.float().double()
+    box = T.cpu().numpy().astype('float32')
+    disp, _ = jmd.space.periodic_general(box)
+    kw['fractional_coordinates'] = True
+  sig = torch.tensor([[1.0, 0.95], [0.95, 0.9]], device=DEV)
   if kind == 'soft':
     nfn, efn = jmd.energy.soft_sphere_neighbor_list(disp, box, sigma=1.2, **kw)
-  elif kind == 'lj':
+  elif kind != 'lj species':
     nfn, efn = jmd.energy.lennard_jones_neighbor_list(disp, box, **kw)
   else:
     species = torch.arange(n, device=DEV, dtype=torch.int32) % 2
@@ -78,6 +86,8 @@ def test_rows_of_a_large_table(kind):
     hi = min(lo + (1 << 23), n)
     j = idx[lo:hi, :6].long()
     d = R[j].double() - R[lo:hi, None].double()
+    if kind == 'lj matrix':
+      d = d @ T.T
     s = (d * d).sum(-1)
     sg = 1.2 if kind == 'soft' else 1.0
     if kind == 'lj species':

@@ -5,6 +5,8 @@ some dimensions only, species parameters and box matrices.  Forces against the f
 the bars of test_gpu_pair.py (float32 pair terms: 1e-5 norm-wise, 5e-5 of the
 rms for one particle, 1e-6 for the energy)."""
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -119,6 +121,43 @@ def test_rows_with_species_and_box_matrix(lanes, species, matrix):
       assert rel <= FORCE_RTOL and worst <= FORCE_WORST
     E, _ = efn.energy_and_force(Rt, nbrs)
     assert abs(float(E) - E64) <= 1e-6 * abs(E64)
+  finally:
+    lib.jmd_set_threads_per_atom(0)
+
+
+@pytest.mark.parametrize('lanes', [0, 2, 4, 8, 16])
+@pytest.mark.parametrize('dim', [2, 3])
+def test_rows_narrower_than_a_block(dim, lanes):
+  """Soft-sphere rows cut to every width around a block of 4 entries a lane
+  (fewer entries than lanes, a full block, one more), some rows ending before."""
+  import jax_md_amd as jmd
+  rng = np.random.default_rng(dim)
+  n, L = 1500, np.float32(30.0 if dim == 2 else 10.0)
+  R = rng.uniform(0, L, (n, dim)).astype(np.float32)
+  disp, _ = jmd.space.periodic(L)
+  nfn, efn = jmd.energy.soft_sphere_neighbor_list(disp, L, sigma=2.0, dr_threshold=0.2,
+                                                  format=jmd.partition.Dense)
+  Rt = torch.as_tensor(R, device=DEV)
+  nbrs = nfn.allocate(Rt)
+  lib = jmd._native.load()
+  assert lib.jmd_set_threads_per_atom(lanes) == 0
+  try:
+    for width in (1, 2, 3, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33):
+      width = min(width, nbrs.idx.shape[1])
+      rows = nbrs.idx[:, :width].contiguous()
+      idx = rows.cpu().numpy()
+      i, k = np.nonzero(idx < n)
+      d = R[idx[i, k]].astype(np.float64) - R[i]
+      d -= float(L) * np.rint(d / float(L))
+      r = np.sqrt((d ** 2).sum(1))
+      g = np.where(r < 2.0, -(1 - r / 2.0) / (2.0 * r), 0.0)
+      F64 = np.zeros((n, dim))
+      np.add.at(F64, i, g[:, None] * d)
+      for in_box in (False, True):
+        F = efn.force(Rt, dataclasses.replace(nbrs, idx=rows), in_box=in_box)
+        rel, worst = _force_err(F.cpu().numpy(), F64)
+        print(f'narrow rows {dim}-D lanes {lanes} width {width}: {rel:.2e} {worst:.2e}', flush=True)
+        assert rel <= FORCE_RTOL and worst <= FORCE_WORST
   finally:
     lib.jmd_set_threads_per_atom(0)
 
