@@ -1166,9 +1166,7 @@ __global__ __launch_bounds__(256) void k_skin_check(const float* __restrict__ po
     load_pos<DIM>(ref, i, b);
     moved = ref_metric_sq<DIM>(a, b, s) > threshold_sq;
   }
-  // one wavefront of the workgroup speaks for all of them
-  moved = __syncthreads_or(moved);
-  if (threadIdx.x < kWave) raise_gate(gate, moved);
+  raise_gate(gate, moved);
 }
 
 // ---------------------------------------------------------------------------

@@ -364,3 +364,32 @@ def test_custom_mask_function_known_answer_and_oracle():
   onl2 = O.neighbor_list_update(spec, R2, onl)
   assert np.array_equal(nb.idx.cpu().numpy(), onl2.idx)
   assert int(nb.error.code) == int(onl2.error)
+
+
+@pytest.mark.parametrize('n', [1, 64, 65, 4096, 300001])
+@pytest.mark.parametrize('dim', [2, 3])
+def test_skin_check_raises_its_word_only(dim, n):
+  """The gate word is raised when any particle moved beyond the threshold,
+  whichever wavefronts see it, stays up when none did, and the words beside
+  it keep their values."""
+  print(f'case skin check dim={dim} n={n}', flush=True)
+  from jax_md_amd import _native as nat
+  lib = nat.load()
+  rng = np.random.default_rng(n)
+  R = torch.as_tensor(rng.uniform(0, 50, (n, dim)).astype(np.float32), device=DEV)
+  ref = R.clone()
+  words = torch.arange(1, 65, dtype=torch.int32, device=DEV)
+  want = words.clone()
+  gate = words[5:]
+  for moved in ((), (0,), (n - 1,), (n // 2,), tuple(range(0, n, 64)), slice(None), ()):
+    X = ref.clone()
+    if moved != ():
+      X[list(moved) if isinstance(moved, tuple) else moved] += 0.5
+    # raised words stay up: the last, closed pass starts from a raised one
+    start = 0 if moved != () or int(want[5]) != 1 else 1
+    words[5] = start
+    nat.check(lib.jmd_neighbor_list_check(
+        nat.ptr(X), dim, nat.ptr(ref), n, dim, 1, nat.f3([50.0] * dim), 0.0625, nat.ptr(gate),
+        nat.stream_handle(R.device)), 'check')
+    want[5] = 1 if moved != () else start
+    assert torch.equal(words, want), (moved if isinstance(moved, slice) else len(moved))
