@@ -345,3 +345,42 @@ def test_x64_trajectory_gradient_long_horizon():
   ad = float(np.sum(g * u))
   print(f'  d/dx0 . u: adjoint {ad:.8e} fd {fd:.8e} |grad| {np.linalg.norm(g):.3e}')
   assert abs(ad - fd) <= 1e-4 * max(abs(fd), np.linalg.norm(g))
+
+
+@pytest.mark.parametrize('dim', [2, 3])
+def test_force_vjp_rows_around_a_batch(dim):
+  """Soft-sphere rows cut to widths around one and two entries a lane, where a
+  lane's second entry exists in some lanes or in none: J v and v^T dF/dsigma
+  (1e-5 of float64, the latter of its terms' magnitudes) row by row."""
+  jmd = _jmd()
+  rng = np.random.default_rng(dim)
+  n, L, sig = 1200, F32(26.0 if dim == 2 else 9.0), 2.0
+  R = rng.uniform(0, L, (n, dim)).astype(F32)
+  v = rng.normal(size=(n, dim)).astype(F32)
+  disp, _ = jmd.space.periodic(L)
+  nfn, efn = jmd.energy.soft_sphere_neighbor_list(disp, L, sigma=sig, dr_threshold=0.2,
+                                                  format=jmd.partition.Dense)
+  Rt = torch.as_tensor(R, device=DEV)
+  nb = nfn.allocate(Rt)
+  for width in (1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33):
+    rows = nb.idx[:, :min(width, nb.idx.shape[1])].contiguous()
+    idx = rows.cpu().numpy()
+    i, k = np.nonzero(idx < n)
+    j = idx[i, k]
+    d = R[j].astype(np.float64) - R[i]
+    d -= float(L) * np.rint(d / float(L))
+    r = np.sqrt((d ** 2).sum(1))
+    ok = r < sig
+    i, j, d, r = i[ok], j[ok], d[ok], r[ok]
+    w = v[j].astype(np.float64) - v[i]
+    g, gp = -(1 - r / sig) / (sig * r), 0.5 / (sig * r ** 3)
+    h = g[:, None] * w + (2 * gp * (d * w).sum(1))[:, None] * d
+    want = np.zeros((n, dim))
+    np.add.at(want, i, h)
+    t = (1 / (sig ** 2 * r) - 2 / sig ** 3) * (v[i] * d).sum(1)
+    Jv, pc, _ = jmd.adjoint.force_vjp(efn, Rt, dataclasses.replace(nb, idx=rows),
+                                      torch.as_tensor(v, device=DEV))
+    rel = np.linalg.norm(Jv.cpu().numpy() - want) / np.linalg.norm(want)
+    print(f'vjp rows {dim}-D width {rows.shape[1]}: {rel:.2e}', flush=True)
+    assert rel <= 1e-5
+    assert abs(float(pc[0]) - t.sum()) <= 1e-5 * np.abs(t).sum()
