@@ -15,7 +15,8 @@
 //   V = 4 eps (s^12 - s^6),  V'/r = -24 eps (2 s^12 - s^6) / r^2,
 //   S = (rc^2 - r^2)^2 (rc^2 + 2 r^2 - 3 ro^2) / (rc^2 - ro^2)^3,
 //   S'/r = 12 (rc^2 - r^2)(ro^2 - r^2) / (rc^2 - ro^2)^3   on [r_on, r_c),
-//   F_i += (S V'/r + S'/r V) (R_j - R_i).
+//   F_i += (S V'/r + S'/r V) (R_j - R_i),
+// the switch written in y = (rc^2 - r^2) / (rc^2 - ro^2) (lj_reduced).
 #include <mutex>
 
 #include "jmd_pair_dense.hpp"

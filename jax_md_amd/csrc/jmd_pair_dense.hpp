@@ -29,13 +29,14 @@ __device__ __forceinline__ rsrc_t row_table(const float* p, unsigned rows, int r
 // Sum over one Dense row slice (entries sub, sub+TPA, ...) into f, e.
 //
 // What bounds it: the gathers, then VALU issue.  A list at r_c + skin = 3.0
-// holds 95 entries a row at rho 0.8442; at N = 262,144 the L1 serves 22 M
-// requests a launch (86 k of 115 k cycles on each CU) and each SIMD issues
-// 80 k cycles of VALU work, 35 operations a pair and 26 of them the pair's
-// own.  (Timing copies: without half of the arithmetic 1.5 us of 49 less, with
-// neighbours that are consecutive rows 12 us less.  16-byte loads of the
-// entries saved a third of the load instructions and made the gathers' L1
-// requests 15% more; two blocks of entries in flight changed nothing.)
+// holds 95 entries a row at rho 0.8442; at N = 262,144 the L1 serves 22.5 M
+// requests a launch (88 k of 114 k cycles on each CU) and each SIMD issues
+// 80 k cycles of VALU work, 52 lane operations an entry with the ends of the
+// rows and the step's epilogue.  (Timing copies: without half of the
+// arithmetic 1.5 us of 49 less, with neighbours that are consecutive rows 12 us
+// less.  16-byte loads of the entries saved a third of the load instructions
+// and made the gathers' L1 requests 15% more; two blocks of entries in flight
+// changed nothing.)
 // * Folds are decided per block of UNR entries and dimension: while every
 //   plain difference of the block is shorter than half the side, it is the
 //   minimum image, and a maximum and a ballot replace the selects.  `near`
