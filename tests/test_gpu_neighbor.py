@@ -393,3 +393,29 @@ def test_skin_check_raises_its_word_only(dim, n):
         nat.stream_handle(R.device)), 'check')
     want[5] = 1 if moved != () else start
     assert torch.equal(words, want), (moved if isinstance(moved, slice) else len(moved))
+
+
+@pytest.mark.parametrize('fmt', [O.DENSE, O.SPARSE])
+@pytest.mark.parametrize('outside', [False, True])
+@pytest.mark.parametrize('dim,L', [(3, 17.0), (3, 40.3), (3, 150.7), (2, 1203.5)])
+def test_pairs_at_the_cutoff_bit_exact(dim, L, outside, fmt):
+  """Pairs whose distance is the list cutoff to within a few roundings of the
+  coordinates, across every face, with positions in the box and up to one
+  period outside: the fast test may not decide any of them differently from
+  the reference's float32 d^2, nor the pruning drop a candidate of a particle
+  below the box, whose cell index is truncated towards zero."""
+  print(f'case cutoff dim={dim} L={L} outside={outside} fmt={fmt}', flush=True)
+  rng = np.random.default_rng(int(L) + dim)
+  n, c = 1500, 3.0
+  a = rng.uniform(0, L, (n, dim))
+  a[:n // 2] = np.where(rng.random((n // 2, dim)) < 0.5, rng.uniform(-2, 2, (n // 2, dim)) % L,
+                        a[:n // 2])  # near the faces
+  e = rng.normal(size=(n, dim))
+  e /= np.linalg.norm(e, axis=1)[:, None]
+  off = rng.uniform(-8, 8, n) * 2.0 ** -24 * (L + c)
+  b = (a + e * (c + off)[:, None]) % L
+  R = np.concatenate([a, b]).astype(F32)
+  if outside:
+    R = (R + F32(L) * rng.integers(-1, 2, size=R.shape).astype(F32)).astype(F32)
+  _, _, g, o = _both(R, F32(L), 2.5, 0.5, fmt)
+  _assert_same(g, o, f'cutoff dim={dim} L={L} outside={outside} fmt={fmt}')
